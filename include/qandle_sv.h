@@ -248,6 +248,54 @@ int qs_compose_tables(float *utab, float *qtab, const int32_t *recipes,
                       const int32_t *offsets, int nrec, const float *cs,
                       void *stream);
 
+/* Everything the passes of one call read besides the state, made in one launch
+ * (QS_SETUP_MAX_NAMED: named inputs it takes):
+ * - cs: (cos, sin) of every half angle, entries 0..nphi) from phi, then B per
+ *   named input (element b at named[j][b * named_stride[j]]).  phi = NULL: cs
+ *   is an input (filled before), and no angle is read;
+ * - utab (and, with qtab, the generators) of the recipes in `words`
+ *   (qs_compose_tables' records): uniform[2i] is the word offset of recipe i
+ *   shared by the batch and uniform[2i + 1] its entry in ltab (-1: none), which
+ *   gets its matrix-core operands (qs_lane_coeffs; of U^dagger with dagger);
+ *   sampled[i] the offsets of the per-sample recipes (B entries each);
+ * - efac (NULL: none): product-state factors (qs_product_factors) with the
+ *   rotations of recipe lead_words + lead[pos] applied (lead[pos] < 0: none;
+ *   lead = NULL: none anywhere); column[pos] is the embedded column of x (row
+ *   stride x_stride, column stride x_step) at bit position pos, -1 for |0>.
+ * Same values as qs_half_angle_coeffs, qs_compose_tables, qs_lane_coeffs,
+ * qs_product_factors and qs_factor_apply one after another.  All pointers are
+ * device memory; the struct itself is read on the host during the call. */
+#define QS_SETUP_MAX_NAMED 24
+typedef struct qs_setup_args {
+  float *cs;
+  float *utab;
+  float *qtab;
+  float *ltab;
+  float *efac;
+  const float *phi;
+  const float *x;
+  const int32_t *words;
+  const int32_t *uniform;
+  const int32_t *sampled;
+  const int32_t *lead_words;
+  const int32_t *lead;
+  const int32_t *column;
+  int64_t B;
+  int64_t x_stride;
+  int64_t x_step;
+  int64_t nphi;
+  int64_t nuniform;
+  int64_t nsampled;
+  int32_t n;
+  int32_t rot;
+  int32_t nnamed;
+  int32_t dagger;
+  const float *named[QS_SETUP_MAX_NAMED];
+  int64_t named_stride[QS_SETUP_MAX_NAMED];
+} qs_setup_args;
+int64_t qs_setup_args_bytes(void);
+int qs_setup(const qs_setup_args *args, void *stream);
+
 /* Matrix-core operands of composed unitaries (utab, 8 floats each): entry e
  * (16 floats, ltab[16 e + 4 r + k]) is what lane row r = lane & 3 of a 4-lane
  * block supplies to v_mfma_f32_4x4x1f32 for the real 4x4 form of U = utab

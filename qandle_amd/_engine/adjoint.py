@@ -29,10 +29,7 @@ def forward(prog, inp):
     grad = _needs_grad(inp)
     R, TB, cm = fused.choose_config(prog, inp, grad)
     if not grad:
-        cs = fused.build_coeffs(prog, inp)
-        efac = fused.product_factors(prog, inp) if (prog.init[0] == "embed" or inp.state is None) else None
-        psi, probs = fused.execute(prog, inp, cs, efac, R, TB, cm=cm, want_state=not prog.measure)
-        return psi, probs
+        return fused.execute(prog, inp, None, None, R, TB, cm=cm, want_state=not prog.measure)
     from . import backward
 
     return backward.run_with_grad(prog, inp, R, TB, cm)

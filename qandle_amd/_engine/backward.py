@@ -61,8 +61,6 @@ class FusedCircuitFn(torch.autograd.Function):
         inp = fused.Inputs(B, batched, phi_param.device, phi_param.detach(), named,
                            None if embed_x is None else embed_x.detach(),
                            None if state is None else state.detach())
-        cs = fused.build_coeffs(prog, inp)
-        efac = fused.product_factors(prog, inp) if (prog.init[0] == "embed" or state is None) else None
         jit_on = fused.use_jit(prog.n, R, TB)
         fold = fused.folds(prog, jit_on)
         pl = fused.get_plan(prog, R, TB, cm, fold)
@@ -76,8 +74,8 @@ class FusedCircuitFn(torch.autograd.Function):
                 return torch.empty_like(psi)
             return None
 
-        psi, probs = fused.execute(prog, inp, cs, efac, R, TB, cm=cm, want_state=True, checkpoints=keep,
-                                   specialise=jit_on, fold=fold)
+        psi, probs, cs = fused._execute(prog, inp, None, None, R, TB, cm=cm, want_state=True, checkpoints=keep,
+                                        specialise=jit_on, fold=fold)
         ctx.prog, ctx.R, ctx.TB, ctx.cm, ctx.B, ctx.names = prog, R, TB, cm, B, names
         ctx.jit, ctx.fold = jit_on, fold
         ctx.ck_index = sorted(ckpts)
@@ -116,20 +114,19 @@ class FusedCircuitFn(torch.autograd.Function):
         ws, nmain = fused.adjoint_words(prog, pl, B, psi.device, embed, ctx.cm)
         embed_rows = len(prog.init[2]) if embed else 0
         total_rows = nrows + embed_rows
-        utab, qtab = fused.compose_tables(ws, cs)
         wb = lib.qs_adjoint_work_bytes(B, n, R, TB, total_rows)
         gpart = torch.empty(max(wb // 4, 1), dtype=torch.float32, device=psi.device)
         npass = len(pl.passes)
         kern = None
-        ltab = None
         if ctx.jit:
             kern = specialised_adjoint(prog, pl, ws, B, embed, seed is not None, ctx.fold)
             ntiles, NS = adjoint_geometry(B, n, R, TB)
-            idx = kern.lane_index_on(psi.device)
-            if idx is not None:  # U^dagger operands of the matrix-core unitaries, step by step
-                ltab = torch.empty(idx.numel() * 16, dtype=torch.float32, device=psi.device)
-                L.check(lib.qs_lane_coeffs(L.ptr(ltab), L.ptr(utab), L.ptr(idx), idx.numel(), 1, st),
-                        "qs_lane_coeffs")
+        # the unitaries, their generators and U^dagger operands (step by step), from the forward's half angles
+        plan = adjoint_setup(prog, pl, ws, kern, B, psi.device, embed)
+        utab, qtab, ltab = (torch.empty(max(c, 1) * w, dtype=torch.float32, device=psi.device)
+                            for c, w in ((plan.nu, 8), (plan.nq, 8), (plan.nlane, 16)))
+        args = plan.fill(B, L.ptr(cs), L.ptr(utab), L.ptr(ltab), qtab=L.ptr(qtab))
+        L.check(lib.qs_setup(L.ctypes.byref(args), st), "qs_setup")
         events = launch_events
         for k, (w, nsub, lpos) in enumerate(ws.passes):
             seed_ptr = None if (k > 0 or seed is None) else L.ptr(seed)
@@ -192,6 +189,16 @@ class FusedCircuitFn(torch.autograd.Function):
             shp = ctx.state_shape
             g_state = lam.sum(0) if len(shp) == 1 else (lam if lam.shape == shp else lam.sum(0, keepdim=True))
         return (None, None, None, None, None, None, None, g_param, g_embed, g_state, *g_named)
+
+
+def adjoint_setup(prog, pl, ws, kern, B, device, embed):
+    """fused.setup_plan of an adjoint sweep's tables, kept with the program."""
+    key = ("setup_adj", id(pl), B, str(device), embed, kern is None)
+    hit = prog.words_cache.get(key)
+    if hit is None:
+        hit = fused.setup_plan(prog, ws, None if kern is None else kern.lane_index, B, device, dagger=True)
+        prog.words_cache[key] = hit
+    return hit
 
 
 def gradient_scatter(prog, rows, device):

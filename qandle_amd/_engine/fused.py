@@ -571,6 +571,7 @@ class WordSet:
     nu: int                       # U entries
     nq: int                       # gradient-generator entries
     host: list = None             # the same passes with their words as host numpy arrays
+    entries: list = None          # (recipe word offset, first U entry, per sample) of every recipe
 
     def host_passes(self):
         """The passes with host words (what the kernel compilers read; no device copy back)."""
@@ -580,7 +581,7 @@ class WordSet:
 def upload_tables(passes, tables: PL.TableBuilder, device, host=None) -> WordSet:
     rec = L.upload(tables.recipes(), torch.int32, device)
     off = L.upload(np.asarray(tables.offsets or [0], dtype=np.int32), torch.int32, device)
-    return WordSet(passes, rec, off, tables.count, tables.nu, tables.nq, host)
+    return WordSet(passes, rec, off, tables.count, tables.nu, tables.nq, host, list(tables.entries))
 
 
 def compose_tables(ws: WordSet, cs: torch.Tensor, generators: bool = True):
@@ -731,12 +732,13 @@ def _leading_tables(prog: Program, per_pos, B: int, device):
         tables = PL.TableBuilder(B)
         unit = np.full(prog.n, -1, dtype=np.int32)
         span = np.ones(prog.n, dtype=np.int32)
+        where = np.full(prog.n, -1, dtype=np.int32)  # recipe's word offset by position (qs_setup)
         for pos in sorted(per_pos):
             u, ps, _ = tables.add([(g.kind, index[g.slot], per_sample[g.slot]) for g in per_pos[pos]])
-            unit[pos], span[pos] = u, (B if ps else 1)
+            unit[pos], span[pos], where[pos] = u, (B if ps else 1), tables.offsets[-1]
         recipes = L.upload(tables.recipes(), torch.int32, device)
         offsets = L.upload(tables.offsets, torch.int32, device)
-        hit = (recipes, offsets, tables.count, tables.nu, unit, span)
+        hit = (recipes, offsets, tables.count, tables.nu, unit, span, L.upload(where, torch.int32, device))
         prog.words_cache[key] = hit
     return hit
 
@@ -746,7 +748,7 @@ def absorb_factors(prog: Program, per_pos, efac: torch.Tensor, cs: torch.Tensor,
     their unitaries are composed per bit position on the device (one recipe
     per position, per sample when an input angle is among them) and applied by
     qs_factor_apply."""
-    recipes, offsets, nrec, nu, unit, span = _leading_tables(prog, per_pos, B, efac.device)
+    recipes, offsets, nrec, nu, unit, span, _ = _leading_tables(prog, per_pos, B, efac.device)
     lib = L.load()
     st = L.stream_of(efac)
     utab = torch.empty(max(nu, 1) * 8, dtype=torch.float32, device=efac.device)
@@ -756,6 +758,87 @@ def absorb_factors(prog: Program, per_pos, efac: torch.Tensor, cs: torch.Tensor,
     L.check(lib.qs_factor_apply(L.ptr(out), L.ptr(efac), L.ptr(utab), nu, L.i32_array(unit), L.i32_array(span),
                                 B, prog.n, st), "qs_factor_apply")
     return out
+
+
+@dataclasses.dataclass
+class SetupPlan:
+    """The call-independent part of a qs_setup launch for one encoded program:
+    its argument block with the recipe and factor index arrays filled in, and the
+    sizes of the tables it writes.  ``keep`` holds those device arrays."""
+
+    args: bytes
+    total: int                # half-angle entries
+    nu: int
+    nq: int
+    nlane: int                # matrix-core operand entries
+    factors: bool
+    keep: tuple
+
+    def fill(self, B, cs, utab, ltab, efac=None, qtab=None):
+        """A call's own argument block with its output tables (device addresses)."""
+        a = L.SetupArgs.from_buffer_copy(self.args)
+        a.B, a.cs, a.utab, a.ltab, a.efac, a.qtab = B, cs, utab, ltab, efac, qtab
+        return a
+
+
+def setup_plan(prog: Program, ws: WordSet, lane_index, B: int, device, lead=None, factors: bool = False,
+               dagger: bool = False) -> SetupPlan:
+    """qs_setup's plan for the recipes of ``ws``: the uniform ones with their entry
+    of ``lane_index`` (jit's lane-table order), the per-sample ones, and with
+    ``factors`` the product-state factors with the leading rotations of ``lead``
+    (their _leading_tables) applied."""
+    slot = {int(u): k for k, u in enumerate(lane_index or [])}
+    uniform, sampled = [], []
+    for off, u, ps in ws.entries:
+        if ps:
+            sampled.append(off)
+        else:
+            uniform += [off, slot.get(u, -1)]
+    _, _, total, name_off = coefficient_layout(prog, B)
+    a = L.SetupArgs()
+    column = [-1] * prog.n
+    if factors and prog.init[0] == "embed":
+        a.rot = prog.init[1]
+        for j, b in enumerate(prog.init[2]):
+            column[b] = j
+    index = L.upload(uniform + sampled + column, torch.int32, device)  # one upload of the three arrays
+    keep = [ws.recipes, index]
+    a.words, a.uniform = L.ptr(ws.recipes), L.ptr(index)
+    a.sampled, a.column = a.uniform + 4 * len(uniform), a.uniform + 4 * (len(uniform) + len(sampled))
+    a.nuniform, a.nsampled, a.n, a.dagger = len(uniform) // 2, len(sampled), prog.n, int(dagger)
+    if factors and lead:
+        keep += [lead[0], lead[6]]
+        a.lead_words, a.lead = L.ptr(lead[0]), L.ptr(lead[6])
+    return SetupPlan(bytes(a), total, ws.nu, ws.nq, len(lane_index or []), factors, tuple(keep))
+
+
+def setup_inputs(a, prog: Program, inp: Inputs):
+    """Puts a call's angle and embedding inputs into its qs_setup argument block;
+    returns the tensors that have to live until the launch."""
+    keep = [inp.phi_param.detach()]
+    names = list(inp.named)
+    if len(names) > L.SETUP_MAX_NAMED:  # one table of all angles
+        named = [inp.named[k].detach() for k in names]
+        keep[0] = torch.cat([keep[0]] + [v.expand(inp.B) if v.dim() == 0 else v for v in named])
+        names = []
+    phi = keep[0]
+    a.nphi = phi.numel()
+    a.phi = L.ptr(phi) if a.nphi else a.cs  # no shared angle: any address (it is not read)
+    a.nnamed = len(names)
+    for j, k in enumerate(names):
+        v = inp.named[k]
+        keep.append(v)
+        a.named[j] = L.ptr(v)
+        a.named_stride[j] = v.stride(0) if v.dim() else 0
+    if a.efac and prog.init[0] == "embed":
+        x = inp.embed_x.detach().to(torch.float32)
+        if x.dim() == 1:
+            x = x.unsqueeze(0)
+        if x.shape[0] != inp.B:
+            x = x.expand(inp.B, -1)
+        keep.append(x)
+        a.x, a.x_stride, a.x_step = L.ptr(x), x.stride(0), x.stride(1)
+    return keep
 
 
 def tiles_of(B: int, n: int, K: int) -> int:
@@ -818,7 +901,7 @@ def warm(prog: Program, B: int, R: int, TB: int, cm: PL.CostModel = None, specia
          device="cuda", want_state: bool = False, input_state: bool = False):
     """Builds, uploads and compiles what execute needs for this program and
     batch (the leading rotations' tables, the plan, the pass words and
-    fused-unitary recipes, the compiled kernels and their lane-table index)
+    fused-unitary recipes, the compiled kernels and the setup launch's plan)
     without launching any work.  A caller that will launch on a busy stream
     (a serving loop) warms ahead, so that execute then does no host work
     that waits for the device.  ``input_state``: the call passes an initial
@@ -828,24 +911,43 @@ def warm(prog: Program, B: int, R: int, TB: int, cm: PL.CostModel = None, specia
     n = prog.n
     jit_on = use_jit(n, R, TB) if specialise is None else specialise
     product = not (prog.init[0] in ("input", "amplitude") and input_state)
+    tables = None
     if product and getattr(config, "ABSORB_LEADING_ROTATIONS", True):
         lead = leading_rotations(prog)
         if lead is not None:
-            _leading_tables(prog, lead[1], B, device)
+            tables = _leading_tables(prog, lead[1], B, device)
             prog = lead[0]
     fold = folds(prog, jit_on) and not want_state
     pl = get_plan(prog, R, TB, cm, fold)
     ws = pass_words(prog, pl, B, device)
-    if jit_on:
-        kern = specialised_kernels(prog, pl, ws, B, product, fold)
-        if kern.lanes == "lds":
-            kern.lane_index_on(device)
+    kern = specialised_kernels(prog, pl, ws, B, product, fold) if jit_on else None
+    forward_setup(prog, pl, ws, _setup_lanes(kern), B, device, tables, product)
+
+
+def _setup_lanes(kern):
+    """Lane-table order qs_setup fills for a program's kernels: none when they take no
+    operands or the whole table (jit.lane_mode)."""
+    return kern.lane_index if kern is not None and kern.lanes == "lds" else None
+
+
+def forward_setup(prog: Program, pl: PL.Plan, ws: WordSet, lane_index, B: int, device, lead, factors) -> SetupPlan:
+    """setup_plan of a forward, kept with the program (per plan, batch and device)."""
+    key = ("setup", id(pl), B, str(device), lane_index is None, lead is None, factors)
+    hit = prog.words_cache.get(key)
+    if hit is None:
+        hit = setup_plan(prog, ws, lane_index, B, device, lead, factors)
+        prog.words_cache[key] = hit
+    return hit
 
 
 def execute(prog: Program, inp: Inputs, cs: torch.Tensor, efac, R: int, TB: int,
             cm: PL.CostModel = None, want_state: bool = True, checkpoints=None, events=None,
             specialise: bool = None, fold: bool = None, out: torch.Tensor = None):
     """Runs every pass.  Returns (state or None, probs or None).
+
+    ``cs``, ``efac``: the half-angle table (build_coeffs) and product-state factors
+    (product_factors) of the inputs; ``cs`` None: both are made here, with every
+    other table of the call, in one launch (qs_setup).
 
     ``checkpoints(i, state)``: called after pass i with the state it wrote; when
     it returns a tensor (same shape), the passes continue in that one and the
@@ -862,6 +964,13 @@ def execute(prog: Program, inp: Inputs, cs: torch.Tensor, efac, R: int, TB: int,
     ``fold``: fold trailing CNOTs into the readout of a measured program
     (readout_fold; compiled kernels only), so that the state left behind is
     the one before those CNOTs; None folds when the state is not wanted."""
+    psi, probs, _ = _execute(prog, inp, cs, efac, R, TB, cm, want_state, checkpoints, events, specialise, fold, out)
+    return psi, probs
+
+
+def _execute(prog: Program, inp: Inputs, cs, efac, R: int, TB: int, cm=None, want_state=True, checkpoints=None,
+             events=None, specialise=None, fold=None, out=None):
+    """execute, and the half-angle table it ran with."""
     from .. import config
 
     n, B = prog.n, inp.B
@@ -873,11 +982,17 @@ def execute(prog: Program, inp: Inputs, cs: torch.Tensor, efac, R: int, TB: int,
         if s.shape[0] != B:
             s = s.expand(B, -1)
         src = s.contiguous()
-    if src is None and efac is not None and checkpoints is None and getattr(config, "ABSORB_LEADING_ROTATIONS", True):
+    own = cs is None  # this call makes its tables
+    lead_tables = None
+    if src is None and (own or efac is not None) and checkpoints is None and getattr(
+            config, "ABSORB_LEADING_ROTATIONS", True):
         # the passes then run the remaining gates from the updated factors (same slots, same cs)
         lead = leading_rotations(prog)
         if lead is not None:
-            efac = absorb_factors(prog, lead[1], efac, cs, B)
+            if own:
+                lead_tables = _leading_tables(prog, lead[1], B, inp.device)
+            else:
+                efac = absorb_factors(prog, lead[1], efac, cs, B)
             prog = lead[0]
     jit_on = use_jit(n, R, TB) if specialise is None else specialise
     fold = folds(prog, jit_on) and (not want_state if fold is None else bool(fold))
@@ -885,8 +1000,21 @@ def execute(prog: Program, inp: Inputs, cs: torch.Tensor, efac, R: int, TB: int,
     ws = pass_words(prog, pl, B, inp.device)
     words = ws.passes
     lib = L.load()
-    st = L.stream_of(cs)
-    utab, _ = compose_tables(ws, cs, generators=False)
+    st = torch.cuda.current_stream(inp.device).cuda_stream
+    kern = specialised_kernels(prog, pl, ws, B, src is None, fold) if jit_on else None
+    ltab = None
+    if own:
+        plan = forward_setup(prog, pl, ws, _setup_lanes(kern), B, inp.device, lead_tables, src is None)
+        cs = torch.empty(max(plan.total, 1), 2, dtype=torch.float32, device=inp.device)
+        n_u, n_l, n_f = max(plan.nu, 1) * 8, max(plan.nlane, 1) * 16, B * n * 4 if plan.factors else 0
+        tabs = torch.empty(n_u + n_l + n_f, dtype=torch.float32, device=inp.device)
+        utab, ltab, efac = tabs, tabs[n_u:], tabs[n_u + n_l:] if plan.factors else None
+        args = plan.fill(B, L.ptr(cs), L.ptr(utab), L.ptr(ltab), None if efac is None else L.ptr(efac))
+        hold = setup_inputs(args, prog, inp)
+        L.check(lib.qs_setup(L.ctypes.byref(args), st), "qs_setup")
+        del hold
+    else:
+        utab, _ = compose_tables(ws, cs, generators=False)
     if out is not None:
         if (out.dtype != torch.complex64 or tuple(out.shape) != (B, 2 ** n) or not out.is_contiguous()
                 or out.device != inp.device):
@@ -895,13 +1023,14 @@ def execute(prog: Program, inp: Inputs, cs: torch.Tensor, efac, R: int, TB: int,
     else:
         psi = torch.empty(B, 2 ** n, dtype=torch.complex64, device=inp.device)
     mpart = probs = None
-    if prog.measure:
+    final = prog.measure and kern is not None and kern.final  # the measuring pass writes the probabilities itself
+    if final:
+        mpart = probs = torch.empty(B, n, dtype=torch.float32, device=inp.device)
+    elif prog.measure:
         wb = (lib.qs_readout_work_bytes if fold else lib.qs_fused_measure_work_bytes)(B, n, R, TB)
         mpart = torch.empty(max(wb // 4, 1), dtype=torch.float32, device=inp.device)
     npass = len(words)
-    kern = specialised_kernels(prog, pl, ws, B, src is None, fold) if jit_on else None
-    ltab = None
-    if kern is not None and kern.lanes:
+    if kern is not None and kern.lanes and (ltab is None or kern.lanes is True):
         # operands of the matrix-core unitaries: every table entry (lanes True), or (lanes "lds") each
         # pass's block of the entries it uses, packed pass after pass; none when no pass uses one
         idx = kern.lane_index_on(inp.device) if kern.lanes == "lds" else None
@@ -941,7 +1070,9 @@ def execute(prog: Program, inp: Inputs, cs: torch.Tensor, efac, R: int, TB: int,
             if nxt is not None:
                 # the caller keeps this pass's output; the next pass reads it and writes nxt
                 psi = nxt
-    if prog.measure and fold:
+    if final:
+        pass
+    elif prog.measure and fold:
         probs = torch.empty(B, n, dtype=torch.float32, device=inp.device)
         L.check(lib.qs_readout_finish(L.ptr(probs), L.ptr(mpart), B, n, R, TB, st), "qs_readout_finish")
     elif prog.measure:
@@ -952,7 +1083,7 @@ def execute(prog: Program, inp: Inputs, cs: torch.Tensor, efac, R: int, TB: int,
                                         lpos.ctypes.data_as(L.ctypes.POINTER(L.ctypes.c_int32)), st),
             "qs_fused_measure_finish",
         )
-    return psi, probs
+    return psi, probs, cs
 
 
 def run(prog: Program, circuit, state, kwargs):

@@ -275,8 +275,12 @@ def pass_source(name: str, words, n: int, R: int, TB: int, lpos, gen: bool, meas
                 prefetch: bool = False, waves: int = None, readout=None, valu_pairs: int = 0,
                 lanes=False, split_pairs: bool = False, lane_off: int = 0, interleave: bool = False,
                 wave_sync: bool = False, stagger: int = 0, stagger_cu: int = 256, direct_store: bool = False,
-                direct_load: bool = False) -> str:
+                direct_load: bool = False, final: bool = False) -> str:
     """HIP source of one specialised forward pass kernel (extern "C" ``name``).
+
+    ``final`` (a measuring pass whose tile holds whole samples, n <= R + TB): the
+    probabilities themselves go to ``A.mpart`` as (B, n), since a sample's only
+    partial is its probability; otherwise partials for the finish kernels.
 
     ``prefetch`` keeps the next tile's HBM loads in flight in registers while
     the current tile computes; ``waves`` caps the registers at that many
@@ -396,7 +400,8 @@ def pass_source(name: str, words, n: int, R: int, TB: int, lpos, gen: bool, meas
         _sub_pass(e, sub, s, len(subs), n, R, TB, multi, gen and s == 0, measure and s == len(subs) - 1, readout,
                   valu_pairs, lanes=lane_k if lanes == "lds" else lanes, interleave=interleave,
                   wave_sync=wave_sync and s + 1 < len(subs) and wave_local(sub, subs[s + 1], TB),
-                  tail=[] if direct_store and s == len(subs) - 1 else None, direct_load=direct_load and s == 0)
+                  tail=[] if direct_store and s == len(subs) - 1 else None, direct_load=direct_load and s == 0,
+                  final=final)
     if direct_store:
         e("    __syncthreads();")
         e("  }")
@@ -748,7 +753,7 @@ def wave_local(a, b, TB: int) -> bool:
 
 
 def _sub_pass(e, sub, s, nsub, n, R, TB, multi, gen, measure, readout=None, valu_pairs=0, pipe=None, lanes=False,
-              interleave=False, wave_sync=False, swz_mask=31, tail=None, direct_load=False):
+              interleave=False, wave_sync=False, swz_mask=31, tail=None, direct_load=False, final=False):
     """One sub-pass.  ``pipe`` (pipelined kernels): a dict; the tile is
     ``buf[boff + i]``, no closing barrier is emitted, and a measurement's
     cross-wave finish is left in ``pipe["finish"]`` for after the caller's
@@ -921,7 +926,7 @@ def _sub_pass(e, sub, s, nsub, n, R, TB, multi, gen, measure, readout=None, valu
     if tail is not None:
         _direct_store(e, sub, phys, R)
         if measure:
-            _measure(e, sub, phys, n, R, TB, multi, readout, pipe)
+            _measure(e, sub, phys, n, R, TB, multi, readout, pipe, final)
         e("    }")
         return
     for j in range(NR):
@@ -930,7 +935,7 @@ def _sub_pass(e, sub, s, nsub, n, R, TB, multi, gen, measure, readout=None, valu
         else:
             e(f"      tile[lb ^ {swj[j]}] = v[{phys[j]}];")
     if measure:  # after the tile writes: the amplitudes' registers are free for the partials
-        _measure(e, sub, phys, n, R, TB, multi, readout, pipe)
+        _measure(e, sub, phys, n, R, TB, multi, readout, pipe, final)
     if pipe is None and wave_sync:
         # the next sub-pass keeps this one's wave-index bits: every wave reads back only the
         # quarter of the tile it wrote, and a wave's LDS operations complete in order
@@ -1007,10 +1012,11 @@ def _parity(var: str, mask: int) -> str:
     return f"(__popcll({var} & {mask}LL) & 1)"
 
 
-def _measure(e, sub, phys, n, R, TB, multi, readout=None, pipe=None):
+def _measure(e, sub, phys, n, R, TB, multi, readout=None, pipe=None, final=False):
     """MeasureProbability partials of the tile: K + 1 per slot by local bit
     (layout of qs_fused_measure_finish) or, with ``readout`` masks, n + 1 per
-    slot by bit position (layout of qs_readout_finish)."""
+    slot by bit position (layout of qs_readout_finish).  ``final``: one slot per
+    sample, whose sums are the probabilities: they go to their places in (B, n)."""
     K = R + TB
     T, NR = 1 << TB, 1 << R
     e("      {")
@@ -1061,12 +1067,17 @@ def _measure(e, sub, phys, n, R, TB, multi, readout=None, pipe=None):
         e(f"        for (int q = 0; q < {W}; ++q) {{ float x = c[q];")
         e(f"          for (int off = 1; off < {1 << wlog}; off <<= 1) x += __shfl_xor(x, off, 64); c[q] = x; }}")
     spt_log = (K - n) if multi else 0
-    e(f"        float *mp = A.mpart + (t << {spt_log}) * {W};")
+    row = n if final else W  # floats per slot
+    if final:  # bit position p is qubit n - 1 - p; the total (and, of a multi-sample tile, its sample bits) has no place
+        dst = [n - 1 - d if d < n else -1 for d in dst]
+    e(f"        float *mp = A.mpart + (t << {spt_log}) * {row};")
     if seglog <= 6:
-        e(f"        if ((tid & {(1 << seglog) - 1}) == 0) {{")
-        e(f"          float *ob = mp + (tid >> {seglog}) * {W};")
+        live = f" && (t << {spt_log}) + (tid >> {seglog}) < A.B" if final else ""
+        e(f"        if ((tid & {(1 << seglog) - 1}) == 0{live}) {{")
+        e(f"          float *ob = mp + (tid >> {seglog}) * {row};")
         for q in range(W):
-            e(f"          ob[{dst[q]}] = c[{q}];")
+            if dst[q] >= 0:
+                e(f"          ob[{dst[q]}] = c[{q}];")
         e("        }")
     else:
         wps = 1 << (seglog - 6)
@@ -1079,7 +1090,8 @@ def _measure(e, sub, phys, n, R, TB, multi, readout=None, pipe=None):
                "          float x = 0.f;",
                f"          for (int k = 0; k < {wps}; ++k) x += red[(sm * {wps} + k) * {W} + q];",
                f"          const int dst[{W}] = {{{', '.join(str(d) for d in dst)}}};",
-               f"          A.mpart[((t << {spt_log}) + sm) * {W} + dst[q]] = x;",
+               f"          {'if (dst[q] >= 0 && (t << %d) + sm < A.B) ' % spt_log if final else ''}"
+               f"A.mpart[((t << {spt_log}) + sm) * {row} + dst[q]] = x;",
                "        }"]
         if pipe is not None:
             pipe["finish"] = fin
@@ -1628,6 +1640,8 @@ class ProgramKernels:
         self.pipelined = bool(pipeline) and n >= R + TB
         self.block = (1 << TB) + ((1 << pipeline) if self.pipelined else 0)
         self.full_grid = grid == "full" and not self.pipelined
+        # the measuring pass writes the probabilities where a tile holds whole samples
+        self.final = measure and n <= R + TB and not (self.pipelined or async_loads or tail_prefetch)
         npass = len(passes)
         self.sources, self.names = [], []
         self.lane_index = []  # utab index of every lane-table entry (lanes == "lds"), pass by pass
@@ -1664,7 +1678,8 @@ class ProgramKernels:
                 self.sources.append(pass_source(nm, words, n, R, TB, lpos, gen_first and i == 0,
                                                 measure and i == npass - 1, prefetch, waves, readout, valu_pairs,
                                                 lanes, split_pairs, lane_off, interleave, wave_sync, stagger,
-                                                direct_store=dstore, direct_load=dload))
+                                                direct_store=dstore, direct_load=dload,
+                                                final=self.final and i == npass - 1))
             plain, one = not (use_tail or use_async or self.pipelined), n >= R + TB  # pass_source's gating
             self.direct.append((plain and one and bool(dload) and not (gen_first and i == 0) and not prefetch,
                                 plain and one and bool(dstore)))

@@ -72,6 +72,8 @@ SIGNATURES = {
     "qs_fused_measure_finish": (I32, [P, P, I64, I32, I32, I32, P, P]),
     "qs_readout_work_bytes": (I64, [I64, I32, I32, I32]),
     "qs_lane_coeffs": (I32, [P, P, P, I64, I32, P]),
+    "qs_setup_args_bytes": (I64, []),
+    "qs_setup": (I32, [P, P]),
     "qs_readout_finish": (I32, [P, P, I64, I32, I32, I32, P]),
     "qs_adjoint_work_bytes": (I64, [I64, I32, I32, I32, I32]),
     "qs_adjoint_pass": (I32, [P, P, I64, I32, I32, I32, P, P, I32, P, P, P, P, I32, P, P]),
@@ -92,6 +94,19 @@ SIGNATURES = {
 }
 
 
+SETUP_MAX_NAMED = 24
+
+
+class SetupArgs(ctypes.Structure):
+    """qs_setup_args (include/qandle_sv.h)."""
+
+    _fields_ = [(k, ctypes.c_void_p) for k in ("cs", "utab", "qtab", "ltab", "efac", "phi", "x", "words", "uniform",
+                                               "sampled", "lead_words", "lead", "column")]
+    _fields_ += [(k, I64) for k in ("B", "x_stride", "x_step", "nphi", "nuniform", "nsampled")]
+    _fields_ += [(k, ctypes.c_int32) for k in ("n", "rot", "nnamed", "dagger")]
+    _fields_ += [("named", ctypes.c_void_p * SETUP_MAX_NAMED), ("named_stride", I64 * SETUP_MAX_NAMED)]
+
+
 def load():
     """Load (once) and return the engine library; raises if it is not built."""
     global _lib
@@ -110,6 +125,8 @@ def load():
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = args
+        if lib.qs_setup_args_bytes() != ctypes.sizeof(SetupArgs):
+            raise EngineError(f"{LIB_PATH} was built from another qandle_sv.h (qs_setup_args differs): build it again")
         _lib = lib
     return _lib
 

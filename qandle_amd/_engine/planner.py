@@ -385,6 +385,7 @@ class TableBuilder:
         self.nq = 0
         self.words: list = []
         self.offsets: list = []
+        self.entries: list = []   # (word offset, first U entry, per sample) of every recipe
 
     def add(self, consts, B: int = None):
         ps = any(c[2] for c in consts)
@@ -393,6 +394,7 @@ class TableBuilder:
         self.nu += span
         self.nq += span * len(consts)
         self.offsets.append(len(self.words))
+        self.entries.append((len(self.words), u, ps))
         self.words.extend([u, span, len(consts), q])
         for c in consts:
             self.words.extend([int(c[0]), int(c[1]), 1 if c[2] else 0])

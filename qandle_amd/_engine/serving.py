@@ -465,13 +465,11 @@ class ServingEngine:
                 kw[prog.init[3]] = x[ch.lo:ch.hi] if x.dim() == 2 else x
             inp = fused.gather_inputs(prog, req.circuit.circuit, None, kw)
             R, TB = kernel_shape(prog.n, req.compiled)
-            cs = fused.build_coeffs(prog, inp)
-            efac = fused.product_factors(prog, inp)
             cm = fused.DEFAULT_COST if req.compiled else fused.INTERPRETED_COST
-            _, probs = fused.execute(prog, inp, cs, efac, R, TB, cm=cm, want_state=False, specialise=req.compiled,
+            _, probs = fused.execute(prog, inp, None, None, R, TB, cm=cm, want_state=False, specialise=req.compiled,
                                      out=psi)
             ch.out = probs
-            ch.keep = (cs, efac)
+            ch.keep = inp
             ev = torch.cuda.Event()
             ev.record(s)
             ch.event = ev

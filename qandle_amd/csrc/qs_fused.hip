@@ -20,6 +20,7 @@
 // (src/qandle/measurements.py:120-123).
 #include <string.h>
 
+#include "qs_compose.h"
 #include "qs_pass_common.h"
 
 namespace qs {
@@ -541,47 +542,6 @@ __global__ void k_factor_entries(float *efac, const float *x, const int32_t *ent
 // Im<lam|P_k|psi> at constituent k's output).  kind >= 8 is a gradient probe:
 // identity rotation with Pauli kind - 8.
 // ---------------------------------------------------------------------------
-struct C2 {
-  double re, im;
-};
-__device__ __forceinline__ C2 cm(C2 a, C2 b) { return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re}; }
-__device__ __forceinline__ C2 ca(C2 a, C2 b) { return {a.re + b.re, a.im + b.im}; }
-__device__ __forceinline__ C2 cc(C2 a) { return {a.re, -a.im}; }
-struct M2 {
-  C2 a, b, c, d;  // [[a, b], [c, d]]
-};
-__device__ __forceinline__ M2 mm(const M2 &x, const M2 &y) {
-  return {ca(cm(x.a, y.a), cm(x.b, y.c)), ca(cm(x.a, y.b), cm(x.b, y.d)),
-          ca(cm(x.c, y.a), cm(x.d, y.c)), ca(cm(x.c, y.b), cm(x.d, y.d))};
-}
-__device__ __forceinline__ M2 mdag(const M2 &x) { return {cc(x.a), cc(x.c), cc(x.b), cc(x.d)}; }
-
-__device__ __forceinline__ M2 rot_matrix(int kind, float c, float s) {
-  const C2 z = {0, 0};
-  if (kind == QS_RX) return {{c, 0}, {0, -s}, {0, -s}, {c, 0}};
-  if (kind == QS_RY) return {{c, 0}, {-s, 0}, {s, 0}, {c, 0}};
-  if (kind == QS_RZ) return {{c, -s}, z, z, {c, s}};
-  return {{1, 0}, z, z, {1, 0}};  // gradient probe
-}
-__device__ __forceinline__ M2 pauli(int p) {
-  const C2 z = {0, 0};
-  if (p == QS_RX) return {z, {1, 0}, {1, 0}, z};
-  if (p == QS_RY) return {z, {0, -1}, {0, 1}, z};
-  return {{1, 0}, z, z, {-1, 0}};
-}
-__device__ __forceinline__ void store_m2(float *o, const M2 &x) {
-  o[0] = (float)x.a.re; o[1] = (float)x.a.im; o[2] = (float)x.b.re; o[3] = (float)x.b.im;
-  o[4] = (float)x.c.re; o[5] = (float)x.c.im; o[6] = (float)x.d.re; o[7] = (float)x.d.im;
-}
-
-__device__ __forceinline__ M2 recipe_rot(const int32_t *w, int k, int64_t b, const float2 *csv, int *p) {
-  const int kind = w[4 + 3 * k], ci = w[5 + 3 * k], cps = w[6 + 3 * k];
-  *p = kind < 8 ? kind : kind - 8;
-  if (kind >= 8) return rot_matrix(-1, 1.f, 0.f);
-  const float2 v = csv[ci + (cps ? b : 0)];
-  return rot_matrix(kind, v.x, v.y);
-}
-
 // Per-lane matrix-core operands of fused unitaries: for v_mfma_f32_4x4x1f32,
 // lane row r = lane & 3 of a 4-lane block supplies A[r][k] of the real 4x4 form
 // of U (or, with dagger, of U^dagger, its transpose).  Entry e (16 floats,
@@ -590,22 +550,7 @@ __global__ void k_lane_coeffs(float *ltab, const float *utab, const int32_t *idx
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < count * 4;
        e += (int64_t)gridDim.x * blockDim.x) {
     const int64_t u = e >> 2;
-    const int r = (int)(e & 3);
-    const float *m = utab + 8 * (idx ? (int64_t)idx[u] : u);
-    const float a = m[0], b = m[1], c = m[2], d = m[3], f = m[5], g = m[6], h = m[7], ee = m[4];
-    float4 o;
-    if (!dagger) {
-      if (r == 0) o = make_float4(a, -b, c, -d);
-      else if (r == 1) o = make_float4(b, a, d, c);
-      else if (r == 2) o = make_float4(ee, -f, g, -h);
-      else o = make_float4(f, ee, h, g);
-    } else {
-      if (r == 0) o = make_float4(a, b, ee, f);
-      else if (r == 1) o = make_float4(-b, a, -f, ee);
-      else if (r == 2) o = make_float4(c, d, g, h);
-      else o = make_float4(-d, c, -h, g);
-    }
-    reinterpret_cast<float4 *>(ltab)[e] = o;
+    reinterpret_cast<float4 *>(ltab)[e] = lane_row(utab + 8 * (idx ? (int64_t)idx[u] : u), (int)(e & 3), dagger);
   }
 }
 
@@ -613,25 +558,12 @@ __global__ void __launch_bounds__(64)
 k_compose(float *utab, float *qtab, const int32_t *words, const int32_t *off, int nrec,
           const float *cs) {
   const float2 *csv = reinterpret_cast<const float2 *>(cs);
+  const auto coef = [csv](int64_t i) { return csv[i]; };
   for (int r = blockIdx.x; r < nrec; r += gridDim.x) {
     const int32_t *w = words + off[r];
-    const int64_t uidx = w[0];
-    const int64_t span = w[1];
-    const int m = w[2];
-    const int64_t qidx = w[3];
-    for (int64_t b = threadIdx.x; b < span; b += blockDim.x) {
-      int p;
-      M2 U = {{1, 0}, {0, 0}, {0, 0}, {1, 0}};
-      for (int k = 0; k < m; ++k) U = mm(recipe_rot(w, k, b, csv, &p), U);
-      store_m2(utab + 8 * (uidx + b), U);
-      if (!qtab) continue;
-      M2 V = {{1, 0}, {0, 0}, {0, 0}, {1, 0}};
-      for (int k = m - 1; k >= 0; --k) {
-        const M2 Rk = recipe_rot(w, k, b, csv, &p);
-        const M2 Q = mm(mm(V, pauli(p)), mdag(V));
-        store_m2(qtab + 8 * (qidx + k * span + b), Q);
-        V = mm(V, Rk);
-      }
+    for (int64_t b = threadIdx.x; b < w[1]; b += blockDim.x) {
+      store_m2(utab + 8 * (w[0] + b), recipe_unitary(w, b, coef));
+      if (qtab) recipe_generators(qtab, w, b, coef);
     }
   }
 }

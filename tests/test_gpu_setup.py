@@ -1,0 +1,100 @@
+"""qs_setup (all tables of a call in one launch) against the kernels that make them one by
+one (qs_half_angle_coeffs, qs_compose_tables, qs_lane_coeffs, qs_product_factors,
+qs_factor_apply), and the probabilities a whole-sample tile's measuring pass writes itself.
+
+Both sides run the same float32 / float64 operations on the same angles; the compiler may
+contract the factor products differently, so factors are compared to 4 ulp of 1 and the
+tables bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+import qandle_amd as qandle
+from oracle import fp64
+from qandle_amd._engine import fused
+from qandle_amd._engine import lib as L
+
+pytestmark = pytest.mark.gpu
+
+
+def _circuit(n, names, rot):
+    layers = [qandle.AngleEmbedding(name="x", qubits=list(range(0, n, 2)), rotation=rot)]
+    for q in range(n):
+        layers.append(qandle.RY(q, theta=torch.tensor(0.3 + q), remapping=None))
+        if q < names:
+            layers.append(qandle.RX(q, name=f"a{q}", remapping=None))
+    layers += [qandle.CNOT(q, (q + 1) % n) for q in range(n)]
+    layers += [qandle.RZ(q, theta=torch.tensor(1.7 - q), remapping=None) for q in range(n)]
+    layers += [qandle.RX(q, name=f"a{q}", remapping=None) for q in range(names)]
+    layers += [qandle.CNOT(q + 1, q) for q in range(n - 1)]
+    layers += [qandle.RY(0, theta=torch.tensor(0.4), remapping=None), qandle.MeasureProbability()]
+    return qandle.Circuit(layers, num_qubits=n)
+
+
+@pytest.mark.parametrize("n,B,names,rot", [(2, 1, 0, "rx"), (5, 65, 1, "rz"), (6, 3, 6, "ry"), (26, 2, 25, "rx")])
+def test_setup_tables(device, n, B, names, rot):
+    if names > L.SETUP_MAX_NAMED:  # more names than the launch takes: narrow states, wide inputs only
+        n = 26
+    circ = _circuit(n, names, rot).to(device)
+    prog = fused.lower_circuit(circ.circuit)
+    gen = torch.Generator().manual_seed(n)
+    kw = {f"a{q}": torch.rand(B, 2, generator=gen).to(device)[:, 0] for q in range(names)}  # strided inputs
+    if names:
+        kw["a0"] = torch.tensor(0.7, device=device)  # one angle for the whole batch
+    kw["x"] = torch.rand((n + 1) // 2, B, generator=gen).to(device).t()
+    inp = fused.gather_inputs(prog, circ.circuit, None, kw)
+    R, TB = fused.choose_shape(n)
+    lead = fused.leading_rotations(prog)
+    pl = fused.get_plan(lead[0], R, TB)
+    ws = fused.pass_words(lead[0], pl, B, device)
+    lanes = sorted({u for _, u, ps in ws.entries if not ps})[::-1]
+    tables = fused._leading_tables(prog, lead[1], B, device)
+    plan = fused.setup_plan(lead[0], ws, lanes, B, device, tables, True)
+    new = lambda c: torch.full((c,), float("nan"), device=device)  # noqa: E731
+    cs, utab, ltab, efac = new(2 * plan.total), new(8 * ws.nu), new(16 * len(lanes)), new(4 * B * n)
+    a = plan.fill(B, L.ptr(cs), L.ptr(utab), L.ptr(ltab), L.ptr(efac))
+    hold = fused.setup_inputs(a, prog, inp)
+    L.check(L.load().qs_setup(L.ctypes.byref(a), L.stream_of(cs)), "qs_setup")
+    cs0 = fused.build_coeffs(prog, inp)
+    utab0, _ = fused.compose_tables(ws, cs0, generators=False)
+    ltab0 = new(16 * len(lanes))
+    idx = torch.tensor(lanes, dtype=torch.int32, device=device)
+    L.check(L.load().qs_lane_coeffs(L.ptr(ltab0), L.ptr(utab0), L.ptr(idx), len(lanes), 0, L.stream_of(cs)), "lanes")
+    efac0 = fused.absorb_factors(prog, lead[1], fused.product_factors(prog, inp), cs0, B)
+    assert torch.equal(cs, cs0.reshape(-1))
+    assert torch.equal(utab, utab0[:8 * ws.nu]) and torch.equal(ltab, ltab0)
+    assert (efac - efac0.reshape(-1)).abs().max().item() <= 4 * 2 ** -24
+    del hold
+    # the adjoint's tables from the half angles
+    aw, _ = fused.adjoint_words(prog, fused.get_plan(prog, R, TB), B, device, False)
+    ap = fused.setup_plan(prog, aw, None, B, device, dagger=True)
+    u1, q1 = new(8 * aw.nu), new(8 * aw.nq)
+    a = ap.fill(B, L.ptr(cs0), L.ptr(u1), L.ptr(u1), qtab=L.ptr(q1))
+    L.check(L.load().qs_setup(L.ctypes.byref(a), L.stream_of(cs)), "qs_setup")
+    u0, q0 = fused.compose_tables(aw, cs0)
+    assert torch.equal(u1, u0[:8 * aw.nu]) and torch.equal(q1, q0[:8 * aw.nq])
+
+
+@pytest.mark.parametrize("n,B", [(2, 1), (3, 257), (5, 65), (8, 1), (8, 33), (11, 3), (12, 5), (13, 2)])
+@pytest.mark.parametrize("ring", [True, False])
+def test_probabilities_written_by_the_measuring_pass(device, n, B, ring):
+    """Widths up to the tile's, batches that leave the last tile part empty; ``ring`` ends the
+    circuit in CNOTs (readout parities), else in rotations (the bits themselves)."""
+    gen = torch.Generator().manual_seed(100 * n + B)
+    x = torch.rand(B, n, generator=gen) * 3
+    th = torch.rand(2 * n, generator=gen) * 6
+    layers = [qandle.AngleEmbedding(name="x", qubits=list(range(n)), rotation="ry")]
+    ops = [("embed", "y", list(range(n)), x.double().numpy())]
+    for d in range(2):
+        for q in range(n):
+            layers.append(qandle.RX(q, theta=th[d * n + q], remapping=None))
+            ops.append(("rx", q, float(th[d * n + q])))
+        if d == 0 or ring:
+            for q in range(n - 1):
+                layers.append(qandle.CNOT(q, q + 1))
+                ops.append(("cnot", q, q + 1))
+    circ = qandle.Circuit(layers + [qandle.MeasureProbability()], num_qubits=n).to(device)
+    ref = fp64.measure_prob(fp64.simulate(n, ops), n)
+    with torch.no_grad():
+        P = circ(x=x.to(device)).cpu().numpy().reshape(B, n)
+    assert np.abs(P - ref).max() < 1e-5
