@@ -357,6 +357,17 @@ int qs_adjoint_pass(float *psi, float *lam, int64_t B, int n, int R, int TB,
 int qs_adjoint_finish(float *out, float *tot, const float *gpart, int rows,
                       int64_t B, int n, int R, int TB, void *stream);
 
+/* Gradients from the sweep's partials, routed to where a call returns them:
+ * group g is half the sum of rows rows[first[g]] .. rows[first[g+1] - 1] of
+ * gpart (NS slots each, sps consecutive ones per sample, as
+ * qs_adjoint_work_bytes lays them out), over all samples into
+ * out[place[2g]] when place[2g+1] is 0, else per sample into
+ * out[place[2g] + b * place[2g+1]]; a group without rows gives zeros.
+ * first, rows (int32) and place (int64) are device arrays. */
+int qs_gradients(float *out, const float *gpart, const int32_t *first,
+                 const int32_t *rows, const int64_t *place, int ngroups,
+                 int64_t B, int64_t NS, int64_t sps, void *stream);
+
 /* ---------------------------------------------------------------------------
  * Work-item form for batches of uneven circuits.  A descriptor is an opaque
  * record (size from the *_desc_bytes query) filled on the host from exactly

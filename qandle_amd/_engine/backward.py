@@ -22,6 +22,9 @@ computed outside the Function).
 """
 from __future__ import annotations
 
+import dataclasses
+
+import numpy as np
 import torch
 
 from .. import config
@@ -117,10 +120,8 @@ class FusedCircuitFn(torch.autograd.Function):
         wb = lib.qs_adjoint_work_bytes(B, n, R, TB, total_rows)
         gpart = torch.empty(max(wb // 4, 1), dtype=torch.float32, device=psi.device)
         npass = len(pl.passes)
-        kern = None
-        if ctx.jit:
-            kern = specialised_adjoint(prog, pl, ws, B, embed, seed is not None, ctx.fold)
-            ntiles, NS = adjoint_geometry(B, n, R, TB)
+        ntiles, NS = adjoint_geometry(B, n, R, TB)
+        kern = specialised_adjoint(prog, pl, ws, B, embed, seed is not None, ctx.fold) if ctx.jit else None
         # the unitaries, their generators and U^dagger operands (step by step), from the forward's half angles
         plan = adjoint_setup(prog, pl, ws, kern, B, psi.device, embed)
         utab, qtab, ltab = (torch.empty(max(c, 1) * w, dtype=torch.float32, device=psi.device)
@@ -156,34 +157,26 @@ class FusedCircuitFn(torch.autograd.Function):
                     psi_src = ckpts[i - 1]
                 else:
                     psi.copy_(ckpts[i - 1])
-        per = torch.empty(max(total_rows, 1), B, dtype=torch.float32, device=psi.device)
-        tot = torch.empty(max(total_rows, 1), dtype=torch.float32, device=psi.device)
-        L.check(lib.qs_adjoint_finish(L.ptr(per), L.ptr(tot), L.ptr(gpart), total_rows, B, n, R, TB, st),
-                "qs_adjoint_finish")
-
-        scatter = gradient_scatter(prog, rows, psi.device)
-        # parameters (shared angles): one row each
-        g_param = None
-        if ctx.needs_input_grad[7]:
-            g_param = torch.zeros(len(prog.param_slots), dtype=torch.float32, device=psi.device)
-            if scatter["param"] is not None:
-                idx, src_rows = scatter["param"]
-                g_param.index_add_(0, idx, tot[src_rows])
-        # named inputs: per-sample rows summed over the gates that use the name
+        # every gradient the call returns, from the partials, in one launch
+        need_param = bool(ctx.needs_input_grad[7])
+        named = tuple((name, len(shape) > 0) for k, (name, shape) in enumerate(zip(ctx.names, ctx.named_shapes))
+                      if ctx.needs_input_grad[10 + k])
+        batched_x = embed and len(ctx.embed_shape) > 1
+        route = gradient_route(prog, rows, B, psi.device, need_param, named, embed, batched_x)
+        grads = torch.empty(route.size, dtype=torch.float32, device=psi.device)
+        if route.ngroups:
+            base = L.ptr(route.index)
+            L.check(lib.qs_gradients(L.ptr(grads), L.ptr(gpart), base + route.first, base + route.rows, base,
+                                     route.ngroups, B, NS, slots_per_sample(B, n, R, TB), st), "qs_gradients")
+        g_param = grads[:len(prog.param_slots)] if need_param else None
         g_named = []
-        for k, name in enumerate(ctx.names):
-            if not ctx.needs_input_grad[10 + k]:
-                g_named.append(None)
-                continue
-            rr = scatter["named"].get(name)
-            gv = per[rr].sum(0) if rr is not None else torch.zeros(B, device=psi.device)
-            shape = ctx.named_shapes[k]
-            g_named.append(gv.sum().reshape(shape) if len(shape) == 0 else gv.reshape(shape))
+        for k, shape in enumerate(ctx.named_shapes):
+            lo = route.named.get(ctx.names[k])
+            g_named.append(None if lo is None else grads[lo] if len(shape) == 0 else grads[lo:lo + B].reshape(shape))
         g_embed = None
         if embed_rows:
-            gx = per[nrows:total_rows].t()  # (B, d), already 1/2 Im<lam|P_j|psi>
-            shp = ctx.embed_shape
-            g_embed = gx.sum(0) if len(shp) == 1 else gx.reshape(shp)
+            lo = route.embed
+            g_embed = grads[lo:lo + embed_rows] if not batched_x else grads[lo:].reshape(ctx.embed_shape)
         g_state = None
         if ctx.needs_input_grad[9] and prog.init[0] != "embed":
             shp = ctx.state_shape
@@ -201,30 +194,70 @@ def adjoint_setup(prog, pl, ws, kern, B, device, embed):
     return hit
 
 
-def gradient_scatter(prog, rows, device):
-    """Index tensors that route gradient rows to angles, uploaded once per program
-    and device: ``param`` = (angle index, row) of the unnamed rotations (None
-    when there are none), ``named`` = rows of each named input's gates."""
-    key = ("grad_scatter", str(device))
+@dataclasses.dataclass
+class GradientRoute:
+    """qs_gradients' index arrays for one set of wanted gradients, in one device
+    tensor (places first; ``first`` and ``rows`` are byte offsets into it), and
+    where each gradient lies in the launch's output: the angles from 0, every
+    named input, the embedded features."""
+
+    index: torch.Tensor
+    first: int
+    rows: int
+    ngroups: int
+    size: int
+    named: dict
+    embed: int
+
+
+def gradient_route(prog, rows, B, device, need_param, named, embed, batched_x) -> GradientRoute:
+    """Route of the gradient rows to the wanted gradients, kept with the program.
+    ``named``: (name, whether it has an entry per sample) of the wanted named
+    inputs; ``embed`` the embedded features (rows after the rotations'),
+    ``batched_x``: as (B, d), else summed over the batch."""
+    key = ("grad_route", B, str(device), need_param, named, embed, batched_x)
     hit = prog.words_cache.get(key)
-    if hit is None:
-        slot_pos = {s_: i for i, s_ in enumerate(prog.param_slots)}
-        param_rows, named = [], {}
-        for gi, g in enumerate(prog.gates):
-            if g.kind == 4:  # CNOT
-                continue
-            sl = prog.slots[g.slot]
-            if sl.kind == "param":
-                param_rows.append((slot_pos[g.slot], rows[gi]))
-            elif sl.kind == "named":
-                named.setdefault(sl.name, []).append(rows[gi])
-        hit = {
-            "param": (L.upload([p for p, _ in param_rows], torch.long, device),
-                      L.upload([r for _, r in param_rows], torch.long, device)) if param_rows else None,
-            "named": {nm: L.upload(rr, torch.long, device) for nm, rr in named.items()},
-        }
-        prog.words_cache[key] = hit
+    if hit is not None:
+        return hit
+    by_slot, by_name = {}, {}
+    for gi, g in enumerate(prog.gates):
+        if g.kind == 4:  # CNOT
+            continue
+        sl = prog.slots[g.slot]
+        if sl.kind == "param":
+            by_slot.setdefault(g.slot, []).append(rows[gi])
+        elif sl.kind == "named":
+            by_name.setdefault(sl.name, []).append(rows[gi])
+    groups, size, where = [], 0, {}  # (rows, first output, stride)
+    if need_param:
+        groups += [(by_slot.get(s_, []), i, 0) for i, s_ in enumerate(prog.param_slots)]
+        size = len(prog.param_slots)
+    for name, per_sample in named:
+        groups.append((by_name.get(name, []), size, 1 if per_sample else 0))
+        where[name] = size
+        size += B if per_sample else 1
+    at = size
+    if embed:
+        d = len(prog.init[2])
+        groups += [([len(rows) + j], at + j, d if batched_x else 0) for j in range(d)]
+        size += d * B if batched_x else d
+    first = np.cumsum([0] + [len(g[0]) for g in groups])
+    flat = [r for g in groups for r in g[0]]
+    place = np.asarray([v for g in groups for v in g[1:]], dtype=np.int64)
+    words = np.concatenate([place.view(np.int32), np.asarray(list(first) + flat, dtype=np.int32)])
+    pad = np.zeros(len(words) % 2, dtype=np.int32)
+    index = L.upload(np.concatenate([words, pad]).view(np.int64), torch.int64, device)
+    hit = GradientRoute(index, 8 * len(place), 8 * len(place) + 4 * len(first), len(groups), size, where, at)
+    prog.words_cache[key] = hit
     return hit
+
+
+def slots_per_sample(B: int, n: int, R: int, TB: int) -> int:
+    """Reduction slots per sample of a gradient row (adjoint_geometry)."""
+    K = R + TB
+    seglog = (n - R) if n < K else TB
+    wlog = min(seglog, 6)
+    return 1 << (seglog - wlog) if n < K else (1 << (n - K)) << (TB - wlog)
 
 
 def adjoint_geometry(B: int, n: int, R: int, TB: int):

@@ -78,6 +78,7 @@ SIGNATURES = {
     "qs_adjoint_work_bytes": (I64, [I64, I32, I32, I32, I32]),
     "qs_adjoint_pass": (I32, [P, P, I64, I32, I32, I32, P, P, I32, P, P, P, P, I32, P, P]),
     "qs_adjoint_finish": (I32, [P, P, P, I32, I64, I32, I32, I32, P]),
+    "qs_gradients": (I32, [P, P, P, P, P, I32, I64, I64, I64, P]),
     "qs_factor_entries": (I32, [P, P, P, I64, P]),
     "qs_pass_desc_bytes": (I64, []),
     "qs_pass_desc": (I32, [P, P, P, P, I64, I32, I32, I32, P, P, I32, P, P, P, P, I32]),

@@ -98,3 +98,33 @@ def test_probabilities_written_by_the_measuring_pass(device, n, B, ring):
     with torch.no_grad():
         P = circ(x=x.to(device)).cpu().numpy().reshape(B, n)
     assert np.abs(P - ref).max() < 1e-5
+
+
+@pytest.mark.parametrize("B,sps,pad", [(1, 1, 0), (3, 1, 61), (257, 1, 3), (5, 2, 6), (65, 64, 0), (2, 128, 0), (3, 4096, 64)])
+def test_gradient_sums_and_routes(device, B, sps, pad):
+    """qs_gradients: shared angles (one row, several rows, none), per-sample inputs with a
+    stride, against float64 sums: one rounding to float32 and double sums of at most 2^16 terms."""
+    NS = B * sps + pad
+    gen = torch.Generator().manual_seed(B + sps)
+    part = torch.randn(7, NS, generator=gen)
+    groups = [([2], 0, 0), ([], 1, 0), ([6, 0, 3], 2, 0), ([1, 5], 3, 1), ([4], 3 + B, 2), ([], 4 + B, 2)]
+    size = 3 + B + 2 * B
+    first = np.cumsum([0] + [len(g[0]) for g in groups])
+    rows = [r for g in groups for r in g[0]]
+    dev = lambda v, t: torch.tensor(v, dtype=t, device=device)  # noqa: E731
+    d_first, d_rows = dev(first.tolist(), torch.int32), dev(rows, torch.int32)
+    place = dev([v for g in groups for v in g[1:]], torch.int64)
+    out = torch.full((size,), float("nan"), device=device)
+    gp = part.to(device)
+    L.check(L.load().qs_gradients(L.ptr(out), L.ptr(gp), L.ptr(d_first), L.ptr(d_rows), L.ptr(place), len(groups), B, NS,
+                                  sps, L.stream_of(out)), "qs_gradients")
+    per = part[:, :B * sps].double().reshape(7, B, sps).sum(2) / 2
+    ref = torch.zeros(size, dtype=torch.float64)
+    for rr, at, stride in groups:
+        v = per[rr].sum(0) if rr else torch.zeros(B, dtype=torch.float64)
+        if stride:
+            ref[at:at + B * stride:stride] = v
+        else:
+            ref[at] = v.sum()
+    err = (out.cpu().double() - ref).abs()
+    assert bool((err <= 2.0 ** -23 * ref.abs() + 1e-11).all()), err.max()
