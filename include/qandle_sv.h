@@ -449,6 +449,51 @@ int qs_jit_launch(void *function, unsigned grid, unsigned block, const void *arg
                   int64_t args_size, void *stream);
 int qs_jit_unload(void *module);
 
+/* The argument blocks of the compiled pass kernels and sweep steps. */
+typedef struct qs_pass_call {
+  float *state;
+  const float *src;
+  const float *utab;
+  const float *cs;
+  const float *efac;
+  float *mpart;
+  const float *ltab;
+  int64_t B;
+  int64_t ntiles;
+  int32_t store;
+  int32_t pad;
+} qs_pass_call;
+typedef struct qs_adjoint_call {
+  float *psi;
+  float *lam;
+  const float *utab;
+  const float *qtab;
+  const float *cs;
+  float *gpart;
+  const float *seed_w;
+  const float *ltab;
+  const float *psi_src;
+  int64_t B;
+  int64_t NS;
+  int64_t ntiles;
+} qs_adjoint_call;
+
+/* Every launch of a compiled forward: qs_setup (setup = NULL: none), then pass
+ * i < npass as functions[i] over grid[i] workgroups of `block` threads, reading
+ * src[i] (NULL: it generates the product state), writing dst[i] when store[i];
+ * call gives the rest (its mpart goes to the last pass only).  The arrays and
+ * structs are host memory, read during the call. */
+int qs_run_forward(const qs_setup_args *setup, int npass, void *const *functions,
+                   const unsigned *grid, unsigned block, const float *const *src,
+                   float *const *dst, const int32_t *store,
+                   const qs_pass_call *call, void *stream);
+/* Every launch of a compiled adjoint sweep: step i reads psi from psi_src[i]
+ * (NULL: call->psi, which every step writes); call->seed_w goes to step 0. */
+int qs_run_adjoint(const qs_setup_args *setup, int nstep, void *const *functions,
+                   const unsigned *grid, unsigned block,
+                   const float *const *psi_src, const qs_adjoint_call *call,
+                   void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -22,7 +22,9 @@ computed outside the Function).
 """
 from __future__ import annotations
 
+import ctypes
 import dataclasses
+import typing
 
 import numpy as np
 import torch
@@ -68,16 +70,8 @@ class FusedCircuitFn(torch.autograd.Function):
         fold = fused.folds(prog, jit_on)
         pl = fused.get_plan(prog, R, TB, cm, fold)
         every = config.CHECKPOINT_GATES if getattr(config, "CHECKPOINT_GATES", None) else default_checkpoint_gates(prog.n)
-        marks = checkpoint_after(prog, pl, every)
-        ckpts = {}
-
-        def keep(i, psi):
-            if i in marks:  # the pass's output stays as the checkpoint; later passes write a new buffer
-                ckpts[i] = psi
-                return torch.empty_like(psi)
-            return None
-
-        psi, probs, cs = fused._execute(prog, inp, None, None, R, TB, cm=cm, want_state=True, checkpoints=keep,
+        ckpts = dict.fromkeys(checkpoint_after(prog, pl, every))  # pass outputs kept for the sweep
+        psi, probs, cs = fused._execute(prog, inp, None, None, R, TB, cm=cm, want_state=True, marks=ckpts,
                                         specialise=jit_on, fold=fold)
         ctx.prog, ctx.R, ctx.TB, ctx.cm, ctx.B, ctx.names = prog, R, TB, cm, B, names
         ctx.jit, ctx.fold = jit_on, fold
@@ -110,63 +104,73 @@ class FusedCircuitFn(torch.autograd.Function):
             seed = gout.to(torch.float32).contiguous()
         else:
             lam.copy_(gout.to(torch.complex64).resolve_conj())
-        pl = fused.get_plan(prog, R, TB, ctx.cm, ctx.fold)
-        rows = fused.rotation_rows(prog)
-        nrows = len(rows)
         embed = prog.init[0] == "embed" and ctx.needs_input_grad[8]
-        ws, nmain = fused.adjoint_words(prog, pl, B, psi.device, embed, ctx.cm)
-        embed_rows = len(prog.init[2]) if embed else 0
-        total_rows = nrows + embed_rows
-        wb = lib.qs_adjoint_work_bytes(B, n, R, TB, total_rows)
-        gpart = torch.empty(max(wb // 4, 1), dtype=torch.float32, device=psi.device)
-        npass = len(pl.passes)
-        ntiles, NS = adjoint_geometry(B, n, R, TB)
-        kern = specialised_adjoint(prog, pl, ws, B, embed, seed is not None, ctx.fold) if ctx.jit else None
-        # the unitaries, their generators and U^dagger operands (step by step), from the forward's half angles
-        plan = adjoint_setup(prog, pl, ws, kern, B, psi.device, embed)
-        utab, qtab, ltab = (torch.empty(max(c, 1) * w, dtype=torch.float32, device=psi.device)
-                            for c, w in ((plan.nu, 8), (plan.nq, 8), (plan.nlane, 16)))
-        args = plan.fill(B, L.ptr(cs), L.ptr(utab), L.ptr(ltab), qtab=L.ptr(qtab))
-        L.check(lib.qs_setup(L.ctypes.byref(args), st), "qs_setup")
+        opts = getattr(config, "SPECIALISE_ADJOINT_OPTIONS", None)
+        call = prog.kept(("adjoint_call", R, TB, ctx.cm.key(), B, psi.device.index, ctx.jit, ctx.fold, embed,
+                          seed is not None, tuple(sorted(opts.items())) if opts else ()),
+                         lambda: _adjoint_call(prog, R, TB, ctx.cm, B, psi.device, ctx.jit, ctx.fold, embed,
+                                               seed is not None))
+        call.tables.use(st, psi.device)
+        ws, kern, NS, ntiles = call.ws, call.kern, call.NS, call.ntiles
+        # the unitaries, their generators and U^dagger operands (step by step), from the forward's half angles,
+        # and the sweep's partials
+        n_u, n_q, n_l, n_g = call.sizes
+        work = torch.empty(n_u + n_q + n_l + n_g, dtype=torch.float32, device=psi.device)
+        utab = L.ptr(work)
+        qtab, ltab, gpart = utab + 4 * n_u, utab + 4 * (n_u + n_q), utab + 4 * (n_u + n_q + n_l)
+        args = call.setup.fill(B, L.ptr(cs), utab, ltab, qtab=qtab)
         events = launch_events
-        for k, (w, nsub, lpos) in enumerate(ws.passes):
-            seed_ptr = None if (k > 0 or seed is None) else L.ptr(seed)
-            if events is not None:
-                ev = (torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True))
-                ev[0].record(torch.cuda.current_stream(psi.device))
-            if kern is not None:
-                kern.launch(k, L.ptr(psi), L.ptr(lam), L.ptr(utab), L.ptr(qtab), L.ptr(cs), L.ptr(gpart), seed_ptr,
-                            B, NS, ntiles, st, None if ltab is None else L.ptr(ltab), L.ptr(psi_src))
-                psi_src = psi
-            else:
-                L.check(
-                    lib.qs_adjoint_pass(
-                        L.ptr(psi), L.ptr(lam), B, n, R, TB,
-                        lpos.ctypes.data_as(L.ctypes.POINTER(L.ctypes.c_int32)), L.ptr(w), nsub,
-                        L.ptr(cs), L.ptr(utab), L.ptr(qtab), L.ptr(gpart), total_rows, seed_ptr, st,
-                    ),
-                    "qs_adjoint_pass",
-                )
-            if events is not None:
-                ev[1].record(torch.cuda.current_stream(psi.device))
-                # psi and lambda are read and written once per step; a seeded step reads psi only
-                events.append((ev[0], ev[1], B * (2 ** n) * (24 if seed_ptr is not None else 32)))
-            i = npass - 1 - k  # forward pass this step undid
-            if k < nmain and (i - 1) in ckpts:
+        npass = len(call.pl.passes)
+        seed_ptr = None if seed is None else L.ptr(seed)
+        if kern is not None and events is None:
+            sources = (ctypes.c_void_p * len(ws.passes))()
+            sources[0] = L.ptr(psi_src)
+            for i in ckpts:  # the step after the one that undoes pass i + 1 starts from pass i's kept output
+                sources[npass - 1 - i] = L.ptr(ckpts[i])
+            block = L.AdjointCall(L.ptr(psi), L.ptr(lam), utab, qtab, L.ptr(cs), gpart, seed_ptr, ltab, None, B, NS, ntiles)
+            L.check(lib.qs_run_adjoint(ctypes.byref(args), len(ws.passes), call.functions, call.grid, kern.block, sources,
+                                       ctypes.byref(block), st), "qs_run_adjoint")
+        else:
+            L.check(lib.qs_setup(ctypes.byref(args), st), "qs_setup")
+            for k, (w, nsub, lpos) in enumerate(ws.passes):
+                seeded = seed_ptr if k == 0 else None
+                if events is not None:
+                    ev = (torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True))
+                    ev[0].record(torch.cuda.current_stream(psi.device))
                 if kern is not None:
-                    psi_src = ckpts[i - 1]
+                    kern.launch(k, L.ptr(psi), L.ptr(lam), utab, qtab, L.ptr(cs), gpart, seeded, B, NS, ntiles, st, ltab,
+                                L.ptr(psi_src))
+                    psi_src = psi
                 else:
-                    psi.copy_(ckpts[i - 1])
+                    L.check(
+                        lib.qs_adjoint_pass(
+                            L.ptr(psi), L.ptr(lam), B, n, R, TB,
+                            lpos.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)), L.ptr(w), nsub,
+                            L.ptr(cs), utab, qtab, gpart, call.rows, seeded, st,
+                        ),
+                        "qs_adjoint_pass",
+                    )
+                if events is not None:
+                    ev[1].record(torch.cuda.current_stream(psi.device))
+                    # psi and lambda are read and written once per step; a seeded step reads psi only
+                    events.append((ev[0], ev[1], B * (2 ** n) * (24 if seeded is not None else 32)))
+                i = npass - 1 - k  # forward pass this step undid
+                if k < call.nmain and (i - 1) in ckpts:
+                    if kern is not None:
+                        psi_src = ckpts[i - 1]
+                    else:
+                        psi.copy_(ckpts[i - 1])
         # every gradient the call returns, from the partials, in one launch
         need_param = bool(ctx.needs_input_grad[7])
         named = tuple((name, len(shape) > 0) for k, (name, shape) in enumerate(zip(ctx.names, ctx.named_shapes))
                       if ctx.needs_input_grad[10 + k])
         batched_x = embed and len(ctx.embed_shape) > 1
-        route = gradient_route(prog, rows, B, psi.device, need_param, named, embed, batched_x)
+        route = gradient_route(prog, B, psi.device, need_param, named, embed, batched_x)
+        route.tables.use(st, psi.device)
         grads = torch.empty(route.size, dtype=torch.float32, device=psi.device)
         if route.ngroups:
             base = L.ptr(route.index)
-            L.check(lib.qs_gradients(L.ptr(grads), L.ptr(gpart), base + route.first, base + route.rows, base,
+            L.check(lib.qs_gradients(L.ptr(grads), gpart, base + route.first, base + route.rows, base,
                                      route.ngroups, B, NS, slots_per_sample(B, n, R, TB), st), "qs_gradients")
         g_param = grads[:len(prog.param_slots)] if need_param else None
         g_named = []
@@ -174,9 +178,9 @@ class FusedCircuitFn(torch.autograd.Function):
             lo = route.named.get(ctx.names[k])
             g_named.append(None if lo is None else grads[lo] if len(shape) == 0 else grads[lo:lo + B].reshape(shape))
         g_embed = None
-        if embed_rows:
+        if embed:
             lo = route.embed
-            g_embed = grads[lo:lo + embed_rows] if not batched_x else grads[lo:].reshape(ctx.embed_shape)
+            g_embed = grads[lo:lo + len(prog.init[2])] if not batched_x else grads[lo:].reshape(ctx.embed_shape)
         g_state = None
         if ctx.needs_input_grad[9] and prog.init[0] != "embed":
             shp = ctx.state_shape
@@ -184,14 +188,42 @@ class FusedCircuitFn(torch.autograd.Function):
         return (None, None, None, None, None, None, None, g_param, g_embed, g_state, *g_named)
 
 
-def adjoint_setup(prog, pl, ws, kern, B, device, embed):
-    """fused.setup_plan of an adjoint sweep's tables, kept with the program."""
-    key = ("setup_adj", id(pl), B, str(device), embed, kern is None)
-    hit = prog.words_cache.get(key)
-    if hit is None:
-        hit = fused.setup_plan(prog, ws, None if kern is None else kern.lane_index, B, device, dagger=True)
-        prog.words_cache[key] = hit
-    return hit
+@dataclasses.dataclass
+class AdjointCall:
+    """The part of an adjoint sweep that its calls share: plan, words, kernels, table
+    sizes and the launch list (for qs_run_adjoint)."""
+
+    pl: typing.Any
+    ws: typing.Any
+    nmain: int
+    kern: typing.Any
+    setup: typing.Any
+    sizes: tuple              # floats of utab, qtab, ltab, the gradient partials
+    rows: int
+    ntiles: int
+    NS: int
+    tables: typing.Any
+    functions: typing.Any = None
+    grid: typing.Any = None
+
+
+def _adjoint_call(prog, R, TB, cm, B, device, jit_on, fold, embed, seeded) -> AdjointCall:
+    n = prog.n
+    pl = fused.get_plan(prog, R, TB, cm, fold)
+    ws, nmain = fused.adjoint_words(prog, pl, B, device, embed, cm)
+    rows = len(fused.rotation_rows(prog)) + (len(prog.init[2]) if embed else 0)
+    ntiles, NS = adjoint_geometry(B, n, R, TB)
+    kern = specialised_adjoint(prog, pl, ws, B, embed, seeded, fold) if jit_on else None
+    plan = fused.setup_plan(prog, ws, None if kern is None else kern.lane_index, B, device, dagger=True)
+    part = L.load().qs_adjoint_work_bytes(B, n, R, TB, rows) // 4
+    call = AdjointCall(pl, ws, nmain, kern, plan, (max(plan.nu, 1) * 8, max(plan.nq, 1) * 8, max(plan.nlane, 1) * 16,
+                                                   max(part, 1)), rows, ntiles, NS,
+                       fused.Resident([*plan.keep, *([w for w, _, _ in ws.passes] if kern is None else [])]))
+    if kern is not None:
+        count = len(ws.passes)
+        call.functions = (ctypes.c_void_p * count)(*[f.value for f in kern.funcs])
+        call.grid = (ctypes.c_uint * count)(*[kern.grid(i, ntiles) for i in range(count)])
+    return call
 
 
 @dataclasses.dataclass
@@ -208,17 +240,20 @@ class GradientRoute:
     size: int
     named: dict
     embed: int
+    tables: typing.Any
 
 
-def gradient_route(prog, rows, B, device, need_param, named, embed, batched_x) -> GradientRoute:
+def gradient_route(prog, B, device, need_param, named, embed, batched_x) -> GradientRoute:
     """Route of the gradient rows to the wanted gradients, kept with the program.
     ``named``: (name, whether it has an entry per sample) of the wanted named
     inputs; ``embed`` the embedded features (rows after the rotations'),
     ``batched_x``: as (B, d), else summed over the batch."""
-    key = ("grad_route", B, str(device), need_param, named, embed, batched_x)
-    hit = prog.words_cache.get(key)
-    if hit is not None:
-        return hit
+    return prog.kept(("grad_route", B, device.index, need_param, named, embed, batched_x),
+                     lambda: _gradient_route(prog, B, device, need_param, named, embed, batched_x))
+
+
+def _gradient_route(prog, B, device, need_param, named, embed, batched_x) -> GradientRoute:
+    rows = fused.rotation_rows(prog)
     by_slot, by_name = {}, {}
     for gi, g in enumerate(prog.gates):
         if g.kind == 4:  # CNOT
@@ -247,9 +282,8 @@ def gradient_route(prog, rows, B, device, need_param, named, embed, batched_x) -
     words = np.concatenate([place.view(np.int32), np.asarray(list(first) + flat, dtype=np.int32)])
     pad = np.zeros(len(words) % 2, dtype=np.int32)
     index = L.upload(np.concatenate([words, pad]).view(np.int64), torch.int64, device)
-    hit = GradientRoute(index, 8 * len(place), 8 * len(place) + 4 * len(first), len(groups), size, where, at)
-    prog.words_cache[key] = hit
-    return hit
+    return GradientRoute(index, 8 * len(place), 8 * len(place) + 4 * len(first), len(groups), size, where, at,
+                         fused.Resident([index]))
 
 
 def slots_per_sample(B: int, n: int, R: int, TB: int) -> int:
@@ -278,13 +312,12 @@ def specialised_adjoint(prog, pl, ws, B, embed, seeded, fold=False):
     from . import jit
 
     opts = getattr(config, "SPECIALISE_ADJOINT_OPTIONS", {}) or {}
-    key = ("jit_adj", id(pl), B, embed, seeded, fold, tuple(sorted(opts.items())))
-    hit = prog.words_cache.get(key)
-    if hit is None:
+
+    def make():
         masks = fused.readout_fold(prog)[1] if fold else None
-        hit = jit.AdjointKernels(ws.host_passes(), prog.n, pl.R, pl.TB, seeded, readout=masks, **opts)
-        prog.words_cache[key] = hit
-    return hit
+        return jit.AdjointKernels(ws.host_passes(), prog.n, pl.R, pl.TB, seeded, readout=masks, **opts)
+
+    return prog.kept(("jit_adj", id(pl), B, embed, seeded, fold, tuple(sorted(opts.items()))), make)
 
 
 def run_with_grad(prog, inp, R, TB, cm=None):

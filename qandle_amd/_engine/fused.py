@@ -9,14 +9,17 @@ executed as a short sequence of ``qs_fused_pass`` launches.
 """
 from __future__ import annotations
 
+import ctypes
 import dataclasses
 import math
+import threading
 import typing
 import weakref
 
 import numpy as np
 import torch
 
+from .. import config, qw_map
 from . import lib as L
 from . import planner as PL
 
@@ -35,6 +38,21 @@ class Slot:
     sign: float = 1.0             # -1: the rotation is inverted (Invert of the module)
 
 
+class Common:
+    """What programs of one structure share: their plans, encoded words, device
+    index tables and kernels, none of which depends on a circuit's parameters.
+    Kept alive by the programs alone (a circuit built again with other angles,
+    a copy, or a request of a known template then plans and encodes nothing)."""
+
+    def __init__(self):
+        self.plans: dict = {}
+        self.cache: dict = {}
+
+
+_COMMON: "weakref.WeakValueDictionary" = weakref.WeakValueDictionary()
+_COMMON_LOCK = threading.Lock()
+
+
 @dataclasses.dataclass
 class Program:
     n: int
@@ -49,6 +67,32 @@ class Program:
     def __post_init__(self):
         self.param_slots = [i for i, s in enumerate(self.slots) if s.kind in ("param", "value")]
         self.named_slots = [i for i, s in enumerate(self.slots) if s.kind == "named"]
+        self.angles = None   # AngleList of the parameters, False: gathered gate by gate
+        self._common = None
+
+    @property
+    def common(self) -> Common:
+        if self._common is None:
+            key = (self.n, tuple([x for g in self.gates for x in (g.kind, g.pos, g.ctrl, g.slot)]),
+                   tuple([x for s in self.slots for x in (s.kind, s.name)]),
+                   tuple(tuple(v) if isinstance(v, list) else v for v in self.init), self.measure, self.post)
+            with _COMMON_LOCK:
+                hit = _COMMON.get(key)
+                if hit is None:
+                    hit = _COMMON[key] = Common()
+            self._common = hit
+        return self._common
+
+    def kept(self, key, make):
+        """Cache entry ``key``: this program's, else the one of its structure, else ``make()``."""
+        hit = self.words_cache.get(key)
+        if hit is None:
+            cache = self.common.cache
+            hit = cache.get(key)
+            if hit is None:
+                hit = cache.setdefault(key, make())
+            self.words_cache[key] = hit
+        return hit
 
 
 def _lower_into(layers, n, mapping, prog_gates, slots, state):
@@ -158,10 +202,11 @@ _PROGRAMS: "weakref.WeakKeyDictionary" = weakref.WeakKeyDictionary()
 
 def lower_circuit(circuit) -> typing.Optional[Program]:
     """Program for a built circuit, or None when a layer is outside the program format."""
+    hit = _PROGRAMS.get(circuit, False)
+    if hit is not False:
+        return hit
     from .. import qcircuit
 
-    if circuit in _PROGRAMS:
-        return _PROGRAMS[circuit]
     n = circuit.num_qubits
     gates: typing.List[PL.Gate] = []
     slots: typing.List[Slot] = []
@@ -252,11 +297,13 @@ def get_plan(prog: Program, R: int, TB: int, cm: PL.CostModel = None, fold: bool
     readout_fold keeps (the trailing CNOTs then live in the readout masks)."""
     cm = cm or DEFAULT_COST
     rf = readout_fold(prog) if fold else None
-    key = (R, TB, None if cm is None else dataclasses.astuple(cm), rf is not None)
+    key = (R, TB, cm.key(), rf is not None)
     pl = prog.plans.get(key)
     if pl is None:
-        gates = prog.gates if rf is None else prog.gates[:rf[0]]
-        pl = PL.plan(prog.n, gates, R, TB, cm)
+        pl = prog.common.plans.get(key)
+        if pl is None:
+            gates = prog.gates if rf is None else prog.gates[:rf[0]]
+            pl = prog.common.plans.setdefault(key, PL.plan(prog.n, gates, R, TB, cm))
         prog.plans[key] = pl
     return pl
 
@@ -284,8 +331,6 @@ UNEVEN_COST = PL.CostModel(budget=1024.0, min_low=4)
 def choose_config(prog: Program, inp, grad: bool = False):
     """(R, TB, cost model) for a call: the autotuned choice when enabled, else
     the defaults for a forward-only call or, with ``grad``, for forward + adjoint."""
-    from .. import config
-
     if getattr(config, "AUTOTUNE", False):
         from . import autotune
 
@@ -469,6 +514,48 @@ def _gather_thetas(thetas, cache=None) -> torch.Tensor:
     return flat.index_select(0, idx)
 
 
+class AngleList:
+    """The parameters of a program whose unnamed rotations all have angles of one
+    shape under one remapping, as most circuits' do: read from the modules'
+    parameter tables and stacked in one launch, with none of the per-gate
+    bookkeeping of the general gather.  What that relies on (the remapping,
+    the shapes, a theta that is a Parameter) is checked on every call."""
+
+    def __init__(self, modules, fn, shape):
+        self.modules, self.fn, self.shape = modules, fn, shape
+        self.fns = [fn] * len(modules)
+        self.tables = [m._parameters for m in modules]
+
+    @classmethod
+    def of(cls, prog):
+        """The list of a program, or False where its angles need the general gather."""
+        slots = [prog.slots[i] for i in prog.param_slots]
+        if not slots or any(s.kind != "param" or s.sign != 1.0 for s in slots):
+            return False
+        modules = [s.module for s in slots]
+        fn = modules[0].remapping
+        if fn not in (qw_map.none, qw_map.tanh) or any("theta" not in m._parameters for m in modules):
+            return False
+        shape = tuple(modules[0].theta.shape)
+        return cls(modules, fn, shape) if shape in ((), (1,)) else False
+
+    def gather(self, device):
+        """(S,) float32 remapped angles on ``device``, or None when the modules changed."""
+        if [m.remapping for m in self.modules] != self.fns:
+            return None
+        try:
+            thetas = [t["theta"] for t in self.tables]
+            # both refuse angles of another shape, unless every one has it
+            phi = torch.cat(thetas) if self.shape else torch.stack(thetas)
+        except (KeyError, TypeError, RuntimeError):
+            return None
+        if phi.dim() != 1 or phi.shape[0] != len(thetas):
+            return None
+        if self.fn is not qw_map.none:
+            phi = self.fn(phi)
+        return phi if phi.dtype == torch.float32 and phi.device == device else phi.to(device=device, dtype=torch.float32)
+
+
 def param_angles(prog: Program, device) -> torch.Tensor:
     """Remapped angles of the program's unnamed rotations, in slot order.
 
@@ -478,8 +565,12 @@ def param_angles(prog: Program, device) -> torch.Tensor:
     their gradients come back through one stack) instead of one launch per
     gate; any other remapping callable is applied per gate.  Fixed angles are
     uploaded once per program and device."""
-    from .. import qw_map
-
+    if prog.angles is None:
+        prog.angles = AngleList.of(prog)
+    if prog.angles:
+        phi = prog.angles.gather(device)
+        if phi is not None:
+            return phi
     params = [prog.slots[i] for i in prog.param_slots]
     if not params:
         return torch.zeros(0, dtype=torch.float32, device=device)
@@ -603,10 +694,10 @@ def _encode(p, gates, pl, index, per_sample, tables, rows=None):
 
 def pass_words(prog: Program, pl: PL.Plan, B: int, device) -> WordSet:
     """Forward words of every pass (cached per plan, batch and device)."""
-    key = (id(pl), B, str(device), "fwd")
-    cached = prog.words_cache.get(key)
-    if cached is not None:
-        return cached
+    return prog.kept((id(pl), B, str(device), "fwd"), lambda: _pass_words(prog, pl, B, device))
+
+
+def _pass_words(prog: Program, pl: PL.Plan, B: int, device) -> WordSet:
     index, per_sample, _, _ = coefficient_layout(prog, B)
     tables = PL.TableBuilder(B)
     out, host = [], []
@@ -614,9 +705,7 @@ def pass_words(prog: Program, pl: PL.Plan, B: int, device) -> WordSet:
         w, nsub, lpos = _encode(p, prog.gates, pl, index.__getitem__, per_sample.__getitem__, tables)
         out.append((L.upload(w, torch.int32, device), nsub, lpos))
         host.append((w, nsub, lpos))
-    ws = upload_tables(out, tables, device, host)
-    prog.words_cache[key] = ws
-    return ws
+    return upload_tables(out, tables, device, host)
 
 
 def embed_grad_gates(prog: Program):
@@ -629,10 +718,10 @@ def adjoint_words(prog: Program, pl: PL.Plan, B: int, device, embed: bool, cm: P
     """Reverse-sweep words: the passes in reverse (rotation rows in program
     order), then, with ``embed``, the probe passes of the embedded bits (rows
     after the rotations).  Returns (WordSet, number of reversed forward passes)."""
-    key = (id(pl), B, str(device), "adj", embed)
-    cached = prog.words_cache.get(key)
-    if cached is not None:
-        return cached
+    return prog.kept((id(pl), B, str(device), "adj", embed), lambda: _adjoint_words(prog, pl, B, device, embed, cm))
+
+
+def _adjoint_words(prog: Program, pl: PL.Plan, B: int, device, embed: bool, cm):
     index, per_sample, _, _ = coefficient_layout(prog, B)
     rows = rotation_rows(prog)
     tables = PL.TableBuilder(B)
@@ -652,9 +741,7 @@ def adjoint_words(prog: Program, pl: PL.Plan, B: int, device, embed: bool, cm: P
                                     lambda gi: row0 + gi)
             out.append((L.upload(w, torch.int32, device), nsub, lpos))
             host.append((w, nsub, lpos))
-    hit = (upload_tables(out, tables, device, host), nmain)
-    prog.words_cache[key] = hit
-    return hit
+    return upload_tables(out, tables, device, host), nmain
 
 
 def build_coeffs(prog: Program, inp: Inputs) -> torch.Tensor:
@@ -717,7 +804,10 @@ def leading_rotations(prog: Program):
             touched.update(g.positions)
             keep.append(g)
         if per_pos and keep:
-            hit = (Program(prog.n, keep, prog.slots, prog.init, prog.measure, prog.post), per_pos)
+            rest = Program(prog.n, keep, prog.slots, prog.init, prog.measure, prog.post)
+            # shared with programs of the same full structure only: its tables hold the leading rotations
+            rest._common = prog.common.cache.setdefault("leading", Common())
+            hit = (rest, per_pos)
     prog.words_cache["leading"] = hit
     return hit
 
@@ -725,9 +815,7 @@ def leading_rotations(prog: Program):
 def _leading_tables(prog: Program, per_pos, B: int, device):
     """Recipes of the leading rotations' per-position unitaries (absorb_factors),
     cached per batch and device."""
-    key = ("leading_tables", B, str(device))
-    hit = prog.words_cache.get(key)
-    if hit is None:
+    def make():
         index, per_sample, _, _ = coefficient_layout(prog, B)
         tables = PL.TableBuilder(B)
         unit = np.full(prog.n, -1, dtype=np.int32)
@@ -738,9 +826,9 @@ def _leading_tables(prog: Program, per_pos, B: int, device):
             unit[pos], span[pos], where[pos] = u, (B if ps else 1), tables.offsets[-1]
         recipes = L.upload(tables.recipes(), torch.int32, device)
         offsets = L.upload(tables.offsets, torch.int32, device)
-        hit = (recipes, offsets, tables.count, tables.nu, unit, span, L.upload(where, torch.int32, device))
-        prog.words_cache[key] = hit
-    return hit
+        return recipes, offsets, tables.count, tables.nu, unit, span, L.upload(where, torch.int32, device)
+
+    return prog.kept(("leading_tables", B, str(device)), make)
 
 
 def absorb_factors(prog: Program, per_pos, efac: torch.Tensor, cs: torch.Tensor, B: int) -> torch.Tensor:
@@ -850,8 +938,6 @@ def tiles_of(B: int, n: int, K: int) -> int:
 
 
 def use_jit(n: int, R: int, TB: int) -> bool:
-    from .. import config
-
     return bool(getattr(config, "SPECIALISE", False))
 
 
@@ -860,19 +946,18 @@ def specialised_kernels(prog: Program, pl: PL.Plan, ws: WordSet, B: int, gen_fir
     """Run-time compiled kernels of this plan's passes (cached on the program);
     with ``fold`` the last pass writes readout partials (readout_fold).
     ``load`` False only compiles them into the code-object cache."""
-    from .. import config
     from . import jit
 
     opts = getattr(config, "SPECIALISE_OPTIONS", {}) or {}
-    key = (id(pl), B, gen_first, prog.measure, fold, tuple(sorted(opts.items())))
-    hit = prog.words_cache.get(("jit",) + key)
-    if hit is None:
+
+    def make():
         masks = readout_fold(prog)[1] if fold else None
-        hit = jit.ProgramKernels(ws.host_passes(), prog.n, pl.R, pl.TB, gen_first, prog.measure, readout=masks,
-                                 load=load, **opts)
-        if load:
-            prog.words_cache[("jit",) + key] = hit
-    return hit
+        return jit.ProgramKernels(ws.host_passes(), prog.n, pl.R, pl.TB, gen_first, prog.measure, readout=masks,
+                                  load=load, **opts)
+
+    if not load:
+        return make()
+    return prog.kept(("jit", id(pl), B, gen_first, prog.measure, fold, tuple(sorted(opts.items()))), make)
 
 
 def forward_kernels(prog: Program, B: int, R: int, TB: int, cm: PL.CostModel = None, device="cpu",
@@ -885,8 +970,6 @@ def forward_kernels(prog: Program, B: int, R: int, TB: int, cm: PL.CostModel = N
     so a worker process can build them ahead of a server that runs them later
     (``load`` False: compile into the code-object cache without loading them
     onto a device)."""
-    from .. import config
-
     if getattr(config, "ABSORB_LEADING_ROTATIONS", True) and prog.init[0] in ("embed", "input"):
         lead = leading_rotations(prog)
         if lead is not None:
@@ -906,8 +989,6 @@ def warm(prog: Program, B: int, R: int, TB: int, cm: PL.CostModel = None, specia
     (a serving loop) warms ahead, so that execute then does no host work
     that waits for the device.  ``input_state``: the call passes an initial
     state (no product-state factors)."""
-    from .. import config
-
     n = prog.n
     jit_on = use_jit(n, R, TB) if specialise is None else specialise
     product = not (prog.init[0] in ("input", "amplitude") and input_state)
@@ -932,12 +1013,8 @@ def _setup_lanes(kern):
 
 def forward_setup(prog: Program, pl: PL.Plan, ws: WordSet, lane_index, B: int, device, lead, factors) -> SetupPlan:
     """setup_plan of a forward, kept with the program (per plan, batch and device)."""
-    key = ("setup", id(pl), B, str(device), lane_index is None, lead is None, factors)
-    hit = prog.words_cache.get(key)
-    if hit is None:
-        hit = setup_plan(prog, ws, lane_index, B, device, lead, factors)
-        prog.words_cache[key] = hit
-    return hit
+    return prog.kept(("setup", id(pl), B, str(device), lane_index is None, lead is None, factors),
+                     lambda: setup_plan(prog, ws, lane_index, B, device, lead, factors))
 
 
 def execute(prog: Program, inp: Inputs, cs: torch.Tensor, efac, R: int, TB: int,
@@ -968,14 +1045,74 @@ def execute(prog: Program, inp: Inputs, cs: torch.Tensor, efac, R: int, TB: int,
     return psi, probs
 
 
-def _execute(prog: Program, inp: Inputs, cs, efac, R: int, TB: int, cm=None, want_state=True, checkpoints=None,
-             events=None, specialise=None, fold=None, out=None):
-    """execute, and the half-angle table it ran with."""
-    from .. import config
+class Resident:
+    """Device tables that calls on any stream read: a tensor is freed for reuse in the
+    order of the streams it is known to, so each new stream is made known to all of them."""
 
+    def __init__(self, tensors):
+        self.tensors = tensors
+        self.streams: set = set()
+
+    def use(self, stream: int, device):
+        if stream not in self.streams:
+            cur = torch.cuda.current_stream(device)
+            for t in self.tensors:
+                if t.is_cuda:
+                    t.record_stream(cur)
+            self.streams.add(stream)
+
+
+@dataclasses.dataclass
+class ForwardCall:
+    """The part of a forward that its calls share: plan, words, kernels, table
+    sizes and the launch list (for qs_run_forward)."""
+
+    pl: PL.Plan
+    ws: WordSet
+    kern: typing.Any
+    setup: SetupPlan
+    final: bool               # the measuring pass writes the probabilities itself
+    sizes: tuple              # floats of utab, ltab, efac, the measurement's partials
+    ntiles: int
+    tables: Resident
+    functions: typing.Any = None
+    grid: typing.Any = None
+    store: typing.Any = None
+
+
+def _forward_call(prog, R, TB, cm, B, device, jit_on, fold, from_state, want_state, lead_tables, tables) -> ForwardCall:
+    pl = get_plan(prog, R, TB, cm, fold)
+    ws = pass_words(prog, pl, B, device)
+    lib = L.load()
+    kern = specialised_kernels(prog, pl, ws, B, not from_state, fold) if jit_on else None
+    plan = forward_setup(prog, pl, ws, _setup_lanes(kern), B, device, lead_tables, not from_state) if tables else None
+    final = prog.measure and kern is not None and kern.final
+    part = 0
+    if prog.measure and not final:
+        part = (lib.qs_readout_work_bytes if fold else lib.qs_fused_measure_work_bytes)(B, prog.n, R, TB) // 4
+    sizes = (0, 0, 0, part) if plan is None else (max(plan.nu, 1) * 8, max(plan.nlane, 1) * 16,
+                                                  B * prog.n * 4 if plan.factors else 0, part)
+    used = [ws.recipes, ws.offsets, *([] if plan is None else plan.keep), *([w for w, _, _ in ws.passes] if kern is None else [])]
+    call = ForwardCall(pl, ws, kern, plan, final, sizes, tiles_of(B, prog.n, R + TB), Resident(used))
+    npass = len(ws.passes)
+    store = [1 if (i + 1 < npass or want_state or not prog.measure) else 0 for i in range(npass)]
+    call.store = (ctypes.c_int32 * npass)(*store)
+    if kern is not None:
+        call.functions = (ctypes.c_void_p * npass)(*[f.value for f in kern.funcs])
+        call.grid = (ctypes.c_uint * npass)(*[kern.grid(i, call.ntiles) for i in range(npass)])
+    return call
+
+
+def _execute(prog: Program, inp: Inputs, cs, efac, R: int, TB: int, cm=None, want_state=True, checkpoints=None,
+             events=None, specialise=None, fold=None, out=None, marks=None):
+    """execute, and the half-angle table it ran with.  ``marks`` (a dict by pass
+    index, values filled in): the passes whose output is kept (the later ones run
+    in another buffer); a gradient's forward passes it, with or without entries,
+    and runs every rotation on the state."""
     n, B = prog.n, inp.B
+    device = inp.device
     src = None
-    if prog.init[0] in ("input", "amplitude") and inp.state is not None:
+    if inp.state is not None and prog.init[0] in ("input", "amplitude"):
         s = inp.state.to(torch.complex64).resolve_conj()
         if s.dim() == 1:
             s = s.unsqueeze(0)
@@ -984,128 +1121,146 @@ def _execute(prog: Program, inp: Inputs, cs, efac, R: int, TB: int, cm=None, wan
         src = s.contiguous()
     own = cs is None  # this call makes its tables
     lead_tables = None
-    if src is None and (own or efac is not None) and checkpoints is None and getattr(
-            config, "ABSORB_LEADING_ROTATIONS", True):
+    if (src is None and (own or efac is not None) and checkpoints is None and marks is None
+            and getattr(config, "ABSORB_LEADING_ROTATIONS", True)):
         # the passes then run the remaining gates from the updated factors (same slots, same cs)
         lead = leading_rotations(prog)
         if lead is not None:
             if own:
-                lead_tables = _leading_tables(prog, lead[1], B, inp.device)
+                lead_tables = _leading_tables(prog, lead[1], B, device)
             else:
                 efac = absorb_factors(prog, lead[1], efac, cs, B)
             prog = lead[0]
     jit_on = use_jit(n, R, TB) if specialise is None else specialise
     fold = folds(prog, jit_on) and (not want_state if fold is None else bool(fold))
-    pl = get_plan(prog, R, TB, cm, fold)
-    ws = pass_words(prog, pl, B, inp.device)
-    words = ws.passes
+    opts = getattr(config, "SPECIALISE_OPTIONS", None)
+    call = prog.kept(("call", R, TB, (cm or DEFAULT_COST).key(), B, device.index, jit_on, fold, src is None, want_state,
+                      lead_tables is None, own, tuple(sorted(opts.items())) if opts else ()),
+                     lambda: _forward_call(prog, R, TB, cm, B, device, jit_on, fold, src is not None, want_state,
+                                           lead_tables, own))
     lib = L.load()
-    st = torch.cuda.current_stream(inp.device).cuda_stream
-    kern = specialised_kernels(prog, pl, ws, B, src is None, fold) if jit_on else None
-    ltab = None
+    st = torch._C._cuda_getCurrentRawStream(device.index)
+    call.tables.use(st, device)
+    kern, ws = call.kern, call.ws
+    n_u, n_l, n_f, n_m = call.sizes
+    work = torch.empty(n_u + n_l + n_f + n_m, dtype=torch.float32, device=device)
+    base = L.ptr(work)
+    mpart = base + 4 * (n_u + n_l + n_f)
+    args = hold = None
     if own:
-        plan = forward_setup(prog, pl, ws, _setup_lanes(kern), B, inp.device, lead_tables, src is None)
-        cs = torch.empty(max(plan.total, 1), 2, dtype=torch.float32, device=inp.device)
-        n_u, n_l, n_f = max(plan.nu, 1) * 8, max(plan.nlane, 1) * 16, B * n * 4 if plan.factors else 0
-        tabs = torch.empty(n_u + n_l + n_f, dtype=torch.float32, device=inp.device)
-        utab, ltab, efac = tabs, tabs[n_u:], tabs[n_u + n_l:] if plan.factors else None
-        args = plan.fill(B, L.ptr(cs), L.ptr(utab), L.ptr(ltab), None if efac is None else L.ptr(efac))
+        utab, ltab, factors = base, base + 4 * n_u, base + 4 * (n_u + n_l) if n_f else None
+        cs = torch.empty(max(call.setup.total, 1), 2, dtype=torch.float32, device=device)
+        args = call.setup.fill(B, L.ptr(cs), utab, ltab, factors)
         hold = setup_inputs(args, prog, inp)
-        L.check(lib.qs_setup(L.ctypes.byref(args), st), "qs_setup")
-        del hold
     else:
-        utab, _ = compose_tables(ws, cs, generators=False)
+        table, _ = compose_tables(ws, cs, generators=False)
+        utab, ltab, factors = L.ptr(table), None, None if efac is None else L.ptr(efac)
+    whole = kern is not None and kern.lanes is True  # a lane table of every entry
+    if whole or (not own and kern is not None and kern.lanes):
+        # operands of the matrix-core unitaries, where qs_setup does not make them: every table entry, or
+        # (lanes "lds") each pass's block of the entries it uses, packed pass after pass; none when no pass uses one
+        if own:
+            L.check(lib.qs_setup(ctypes.byref(args), st), "qs_setup")
+            args = None
+        idx = kern.lane_index_on(device) if kern.lanes == "lds" else None
+        if whole or idx is not None:
+            count = ws.nu if idx is None else idx.numel()
+            lanes = torch.empty(max(count, 1) * 16, dtype=torch.float32, device=device)
+            ltab = L.ptr(lanes)
+            L.check(lib.qs_lane_coeffs(ltab, utab, None if idx is None else L.ptr(idx), count, 0, st), "qs_lane_coeffs")
     if out is not None:
         if (out.dtype != torch.complex64 or tuple(out.shape) != (B, 2 ** n) or not out.is_contiguous()
-                or out.device != inp.device):
-            raise ValueError(f"out must be a contiguous ({B}, {2 ** n}) complex64 tensor on {inp.device}")
+                or out.device != device):
+            raise ValueError(f"out must be a contiguous ({B}, {2 ** n}) complex64 tensor on {device}")
         psi = out
     else:
-        psi = torch.empty(B, 2 ** n, dtype=torch.complex64, device=inp.device)
-    mpart = probs = None
-    final = prog.measure and kern is not None and kern.final  # the measuring pass writes the probabilities itself
-    if final:
-        mpart = probs = torch.empty(B, n, dtype=torch.float32, device=inp.device)
-    elif prog.measure:
-        wb = (lib.qs_readout_work_bytes if fold else lib.qs_fused_measure_work_bytes)(B, n, R, TB)
-        mpart = torch.empty(max(wb // 4, 1), dtype=torch.float32, device=inp.device)
-    npass = len(words)
-    if kern is not None and kern.lanes and (ltab is None or kern.lanes is True):
-        # operands of the matrix-core unitaries: every table entry (lanes True), or (lanes "lds") each
-        # pass's block of the entries it uses, packed pass after pass; none when no pass uses one
-        idx = kern.lane_index_on(inp.device) if kern.lanes == "lds" else None
-        if kern.lanes is True or idx is not None:
-            count = ws.nu if idx is None else idx.numel()
-            ltab = torch.empty(max(count, 1) * 16, dtype=torch.float32, device=inp.device)
-            L.check(lib.qs_lane_coeffs(L.ptr(ltab), L.ptr(utab), None if idx is None else L.ptr(idx), count, 0,
-                                       st), "qs_lane_coeffs")
-    ntiles = tiles_of(B, n, R + TB)
-    for i, (w, nsub, lpos) in enumerate(words):
-        last = i == npass - 1
-        store = 1 if (not last or want_state or not prog.measure) else 0
-        if events is not None:
-            ev = (torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True))
-            ev[0].record(torch.cuda.current_stream(inp.device))
-        if kern is not None:
-            kern.launch(i, L.ptr(psi), None if src is None else L.ptr(src), L.ptr(utab), L.ptr(cs),
-                        None if efac is None else L.ptr(efac),
-                        L.ptr(mpart) if (last and mpart is not None) else None, B, ntiles, store, st,
-                        None if ltab is None else L.ptr(ltab))
-        else:
-            L.check(
-                lib.qs_fused_pass(
-                    L.ptr(psi), None if src is None else L.ptr(src), B, n, R, TB,
-                    lpos.ctypes.data_as(L.ctypes.POINTER(L.ctypes.c_int32)), L.ptr(w), nsub,
-                    L.ptr(cs), L.ptr(utab), None if efac is None else L.ptr(efac),
-                    L.ptr(mpart) if (last and mpart is not None) else None, store, st,
-                ),
-                "qs_fused_pass",
-            )
-        if events is not None:
-            ev[1].record(torch.cuda.current_stream(inp.device))
-            events.append(ev)
-        src = psi
-        if checkpoints is not None:
-            nxt = checkpoints(i, psi)
+        psi = torch.empty(B, 2 ** n, dtype=torch.complex64, device=device)
+    probs = torch.empty(B, n, dtype=torch.float32, device=device) if prog.measure else None
+    if call.final:
+        mpart = L.ptr(probs)
+    npass = len(ws.passes)
+    if kern is not None and events is None and checkpoints is None:
+        srcs, dsts = (ctypes.c_void_p * npass)(), (ctypes.c_void_p * npass)()
+        at = None if src is None else L.ptr(src)
+        for i in range(npass):
+            srcs[i], dsts[i] = at, L.ptr(psi)
+            at = dsts[i]
+            if marks and i in marks:  # this output stays; the later passes read it and run in another buffer
+                marks[i] = psi
+                psi = torch.empty_like(psi)
+        block = L.PassCall(None, None, utab, L.ptr(cs), factors, mpart if prog.measure else None, ltab, B, call.ntiles)
+        L.check(lib.qs_run_forward(None if args is None else ctypes.byref(args), npass, call.functions, call.grid,
+                                   kern.block, srcs, dsts, call.store, ctypes.byref(block), st), "qs_run_forward")
+    else:
+        if args is not None:
+            L.check(lib.qs_setup(ctypes.byref(args), st), "qs_setup")
+        for i, (w, nsub, lpos) in enumerate(ws.passes):
+            last = i == npass - 1
+            part = mpart if (last and prog.measure) else None
+            if events is not None:
+                ev = (torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True))
+                ev[0].record(torch.cuda.current_stream(device))
+            if kern is not None:
+                kern.launch(i, L.ptr(psi), None if src is None else L.ptr(src), utab, L.ptr(cs), factors, part, B,
+                            call.ntiles, call.store[i], st, ltab)
+            else:
+                L.check(
+                    lib.qs_fused_pass(
+                        L.ptr(psi), None if src is None else L.ptr(src), B, n, R, TB,
+                        lpos.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)), L.ptr(w), nsub,
+                        L.ptr(cs), utab, factors, part, call.store[i], st,
+                    ),
+                    "qs_fused_pass",
+                )
+            if events is not None:
+                ev[1].record(torch.cuda.current_stream(device))
+                events.append(ev)
+            src = psi
+            nxt = None
+            if marks and i in marks:
+                marks[i] = psi
+                nxt = torch.empty_like(psi)
+            elif checkpoints is not None:
+                nxt = checkpoints(i, psi)
             if nxt is not None:
                 # the caller keeps this pass's output; the next pass reads it and writes nxt
                 psi = nxt
-    if final:
+    del hold
+    if call.final:
         pass
     elif prog.measure and fold:
-        probs = torch.empty(B, n, dtype=torch.float32, device=inp.device)
-        L.check(lib.qs_readout_finish(L.ptr(probs), L.ptr(mpart), B, n, R, TB, st), "qs_readout_finish")
+        L.check(lib.qs_readout_finish(L.ptr(probs), mpart, B, n, R, TB, st), "qs_readout_finish")
     elif prog.measure:
-        probs = torch.empty(B, n, dtype=torch.float32, device=inp.device)
-        lpos = words[-1][2]
+        lpos = ws.passes[-1][2]
         L.check(
-            lib.qs_fused_measure_finish(L.ptr(probs), L.ptr(mpart), B, n, R, TB,
-                                        lpos.ctypes.data_as(L.ctypes.POINTER(L.ctypes.c_int32)), st),
+            lib.qs_fused_measure_finish(L.ptr(probs), mpart, B, n, R, TB,
+                                        lpos.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)), st),
             "qs_fused_measure_finish",
         )
     return psi, probs, cs
 
 
+_adjoint = None
+
+
 def run(prog: Program, circuit, state, kwargs):
     """Forward of a lowered circuit (with the adjoint backward when gradients are needed)."""
-    from .. import measurements
+    global _adjoint
+    if _adjoint is None:
+        from . import adjoint
 
+        _adjoint = adjoint
     inp = gather_inputs(prog, circuit, state, kwargs)
-    from . import adjoint
-
-    out_state, probs = adjoint.forward(prog, inp)
+    out_state, probs = _adjoint.forward(prog, inp)
     if prog.measure:
-        P = probs
-        return measurements.reference_shape(P) if not inp.batched else _batched_probs(P)
+        if probs.shape[0] > 1 and prog.n > 1:
+            return probs  # reference_shape's squeeze has nothing to take
+        from .. import measurements
+
+        return measurements.reference_shape(probs)
     out = out_state if inp.batched else out_state.squeeze(0)
     if prog.post == "abs2":
         from .plain import Abs2Fn
 
         out = Abs2Fn.apply(out)
     return out
-
-
-def _batched_probs(P: torch.Tensor) -> torch.Tensor:
-    from .. import measurements
-
-    return measurements.reference_shape(P)

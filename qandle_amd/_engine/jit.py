@@ -1706,16 +1706,19 @@ class ProgramKernels:
             self._lane_idx[key] = t
         return t
 
+    def grid(self, i: int, ntiles: int) -> int:
+        """Workgroups of pass i's launch."""
+        if self.full_grid and not self.persistent[i]:
+            return max(1, min(ntiles, 0x7fffffff))
+        if self.grid_cap[i] is None:
+            g = L.load().qs_jit_resident_blocks(self.funcs[i], self.block)
+            self.grid_cap[i] = int(g) if g and g > 0 else 2048
+        return max(1, min(ntiles, self.grid_cap[i]))
+
     def launch(self, i: int, state, src, utab, cs, efac, mpart, B: int, ntiles: int, store: int, stream,
                ltab=None):
         lib = L.load()
-        if self.full_grid and not self.persistent[i]:
-            grid = max(1, min(ntiles, 0x7fffffff))
-        else:
-            if self.grid_cap[i] is None:
-                g = lib.qs_jit_resident_blocks(self.funcs[i], self.block)
-                self.grid_cap[i] = int(g) if g and g > 0 else 2048
-            grid = max(1, min(ntiles, self.grid_cap[i]))
+        grid = self.grid(i, ntiles)
         args = struct.pack(ARGS_FMT, state or 0, src or 0, utab or 0, cs or 0, efac or 0, mpart or 0, ltab or 0,
                            B, ntiles, store, 0)
         buf = ctypes.create_string_buffer(args, len(args))
@@ -1777,17 +1780,20 @@ class AdjointKernels:
             cache[key] = L.upload(self.lane_index, torch.int32, device)
         return cache[key]
 
+    def grid(self, i: int, ntiles: int) -> int:
+        """Workgroups of step i's launch."""
+        if self.full_grid:
+            return max(1, min(ntiles, 0x7fffffff))
+        if self.grid_cap[i] is None:
+            g = L.load().qs_jit_resident_blocks(self.funcs[i], self.block)
+            self.grid_cap[i] = int(g) if g and g > 0 else 2048
+        return max(1, min(ntiles, self.grid_cap[i]))
+
     def launch(self, i: int, psi, lam, utab, qtab, cs, gpart, seed_w, B: int, NS: int, ntiles: int, stream,
                ltab=None, psi_src=None):
         """``psi_src``: where the step reads psi (None: psi itself); it writes psi."""
         lib = L.load()
-        if self.full_grid:
-            grid = max(1, min(ntiles, 0x7fffffff))
-        else:
-            if self.grid_cap[i] is None:
-                g = lib.qs_jit_resident_blocks(self.funcs[i], self.block)
-                self.grid_cap[i] = int(g) if g and g > 0 else 2048
-            grid = max(1, min(ntiles, self.grid_cap[i]))
+        grid = self.grid(i, ntiles)
         args = struct.pack(ADJ_FMT, psi, lam, utab or 0, qtab or 0, cs or 0, gpart, seed_w or 0, ltab or 0,
                            psi_src or psi, B, NS, ntiles)
         buf = ctypes.create_string_buffer(args, len(args))

@@ -67,6 +67,8 @@ SIGNATURES = {
     "qs_jit_resident_blocks": (I64, [P, I32]),
     "qs_jit_launch": (I32, [P, ctypes.c_uint, ctypes.c_uint, P, I64, P]),
     "qs_jit_unload": (I32, [P]),
+    "qs_run_forward": (I32, [P, I32, P, P, ctypes.c_uint, P, P, P, P, P]),
+    "qs_run_adjoint": (I32, [P, I32, P, P, ctypes.c_uint, P, P, P]),
     "qs_compose_tables": (I32, [P, P, P, P, I32, P, P]),
     "qs_fused_measure_work_bytes": (I64, [I64, I32, I32, I32]),
     "qs_fused_measure_finish": (I32, [P, P, I64, I32, I32, I32, P, P]),
@@ -108,6 +110,20 @@ class SetupArgs(ctypes.Structure):
     _fields_ += [("named", ctypes.c_void_p * SETUP_MAX_NAMED), ("named_stride", I64 * SETUP_MAX_NAMED)]
 
 
+class PassCall(ctypes.Structure):
+    """qs_pass_call (include/qandle_sv.h)."""
+
+    _fields_ = [(k, ctypes.c_void_p) for k in ("state", "src", "utab", "cs", "efac", "mpart", "ltab")]
+    _fields_ += [("B", I64), ("ntiles", I64), ("store", ctypes.c_int32), ("pad", ctypes.c_int32)]
+
+
+class AdjointCall(ctypes.Structure):
+    """qs_adjoint_call (include/qandle_sv.h)."""
+
+    _fields_ = [(k, ctypes.c_void_p) for k in ("psi", "lam", "utab", "qtab", "cs", "gpart", "seed_w", "ltab", "psi_src")]
+    _fields_ += [("B", I64), ("NS", I64), ("ntiles", I64)]
+
+
 def load():
     """Load (once) and return the engine library; raises if it is not built."""
     global _lib
@@ -141,11 +157,12 @@ def check(status: int, what: str) -> None:
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """Handle of the current stream of a tensor's device (without building a Stream object)."""
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def require_device(t: torch.Tensor, what: str = "tensor") -> None:
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise EngineError(
             f"qandle_amd runs on the MI355X HIP engine only; {what} is on {t.device}. "
             "Move the circuit and its inputs to a HIP device (module.to('cuda'))."

@@ -94,6 +94,10 @@ class CostModel:
     min_low: int = 5            # positions 0..min_low-1 are always local
     lookahead: bool = False     # choose each pass's local positions by the score of the whole schedule
 
+    def key(self) -> tuple:
+        """Its values, as a dictionary key."""
+        return tuple(self.__dict__.values())
+
 
 def _gate_cost(g: Gate, in_regs: bool, cm: CostModel) -> float:
     if g.kind == CNOT:

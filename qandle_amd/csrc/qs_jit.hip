@@ -124,6 +124,46 @@ int qs_jit_launch(void *function, unsigned grid, unsigned block, const void *arg
                                         nullptr, config));
 }
 
+// One call for a program's launches: the tables, then every pass (or sweep step)
+// in stream order.  Enqueueing a pass from the host language costs its argument
+// packing and call besides the launch (9 us each from Python against 4 us here).
+int qs_run_forward(const qs_setup_args *setup, int npass, void *const *functions, const unsigned *grid, unsigned block,
+                   const float *const *src, float *const *dst, const int32_t *store, const qs_pass_call *call,
+                   void *stream) {
+  if (npass < 0 || !call || (npass > 0 && (!functions || !grid || !src || !dst || !store))) return QS_EINVAL;
+  if (setup) {
+    const int rc = qs_setup(setup, stream);
+    if (rc) return rc;
+  }
+  for (int i = 0; i < npass; ++i) {
+    qs_pass_call a = *call;
+    a.state = dst[i];
+    a.src = src[i];
+    a.store = store[i];
+    if (i + 1 < npass) a.mpart = nullptr;
+    const int rc = qs_jit_launch(functions[i], grid[i], block, &a, (int64_t)sizeof(a), stream);
+    if (rc) return rc;
+  }
+  return QS_OK;
+}
+
+int qs_run_adjoint(const qs_setup_args *setup, int nstep, void *const *functions, const unsigned *grid, unsigned block,
+                   const float *const *psi_src, const qs_adjoint_call *call, void *stream) {
+  if (nstep < 0 || !call || (nstep > 0 && (!functions || !grid || !psi_src))) return QS_EINVAL;
+  if (setup) {
+    const int rc = qs_setup(setup, stream);
+    if (rc) return rc;
+  }
+  for (int i = 0; i < nstep; ++i) {
+    qs_adjoint_call a = *call;
+    a.psi_src = psi_src[i] ? psi_src[i] : a.psi;
+    if (i > 0) a.seed_w = nullptr;
+    const int rc = qs_jit_launch(functions[i], grid[i], block, &a, (int64_t)sizeof(a), stream);
+    if (rc) return rc;
+  }
+  return QS_OK;
+}
+
 int qs_jit_unload(void *module) {
   if (!module) return QS_EINVAL;
   return save_hip(hipModuleUnload((hipModule_t)module));
