@@ -339,26 +339,58 @@ def choose_config(prog: Program, inp, grad: bool = False):
             with torch.no_grad():
                 hit, _ = autotune.tune(prog, inp)
         return hit
-    R, TB = choose_shape(prog.n, grad)
+    R, TB = choose_shape(prog.n, grad, inp.B if getattr(config, "SPECIALISE", False) else None)
     return R, TB, (GRAD_COST if grad else DEFAULT_COST)
 
 
-def choose_shape(n: int, grad: bool = False):
-    """(R, TB) of the specialised kernels for a circuit width.
+def choose_shape(n: int, grad: bool = False, B: int = None):
+    """(R, TB) of the specialised kernels for a circuit width and, with ``B``, a batch.
 
     Forward only: from 13 qubits, tiles of 2^13 amplitudes over 256 threads
     with 32 amplitudes per thread (the fewest passes).  With gradients: from
     12 qubits, 2^12-amplitude tiles with 16 amplitudes per thread (the adjoint
     holds psi and lambda, and this shape keeps two waves per SIMD).  From 5
     qubits, 2^11-amplitude tiles of one wave; below that, every bit in
-    registers of a 256-thread tile holding several samples."""
-    if n >= 13 and not grad:
-        return 5, 8
-    if n >= 12:
-        return 4, 8
-    if n >= 5:
-        return 5, 6
-    return n, DEFAULT_TB
+    registers of a 256-thread tile holding several samples.
+
+    Those shapes need a state that fills the chip: 2^20 amplitudes at 32 per
+    thread are 512 waves for 1024 SIMDs.  Below that the time of a pass is the
+    chain of one wave's unitaries (2^(R-1) pairs each), so fewer amplitudes
+    per thread spread it over more waves, at the price of more sub-passes and,
+    past the tile's width, of more passes.  Measured device time of whole
+    calls, old shape -> this one: 8 qubits x 32 forward 23.6 -> 18.4 us, with
+    gradients 112 -> 51; 11 x 75 29.5 -> 23.0 and 138 -> 83; 14 x 4 46 -> 36
+    and 152 -> 120; 16 x 12 64 -> 55 and 215 -> 202; 13 x 200 with gradients
+    (one 2^13 tile per sample) 221 -> 169.  Where the lines lie, both sides:
+    10 x 3000 (2^21.6) R = 3 41.2, R = 4 36.5 us; 16 x 50 (2^21.6) forward
+    R = 4 106.0, R = 5 107.3; 18 x 8 (2^21) with gradients, ladder circuit,
+    R = 3 277, R = 4 258."""
+    if B is None or n < 5:
+        if n >= 13 and not grad:
+            return 5, 8
+        if n >= 12:
+            return 4, 8
+        if n >= 5:
+            return 5, 6
+        return n, DEFAULT_TB
+    amps = B << n
+    if n <= 11:
+        if amps >= 1 << 20:
+            return (5, 6) if n == 11 and not grad else (4, 8)
+        if grad:
+            return (2, 6) if n <= 8 else (3, n - 3)
+        return (3, 8) if n == 11 else (3, 7)
+    if n == 12:
+        return (3, 9) if grad and amps < 1 << 20 else (4, 8)
+    if n == 13:
+        if not grad:
+            return 5, 8
+        return (3, 8) if amps < 1 << 19 else (3, 9) if amps < 1 << 20 else (4, 9)
+    if amps < 1 << 19:
+        return 3, 8
+    if grad:
+        return (3, 9) if amps < 1 << 21 else (4, 8)
+    return (4, 8) if amps < 1 << 20 else (4, 9) if amps < 1 << 22 else (5, 8)
 
 
 def interpreted_shape(n: int):

@@ -128,3 +128,40 @@ def test_gradient_sums_and_routes(device, B, sps, pad):
             ref[at] = v.sum()
     err = (out.cpu().double() - ref).abs()
     assert bool((err <= 2.0 ** -23 * ref.abs() + 1e-11).all()), err.max()
+
+
+@pytest.mark.parametrize("n", [5, 8, 9, 10, 11, 12, 13, 14])
+def test_shapes_of_small_and_full_batches_agree(device, n):
+    """choose_shape's sides of its lines: a few samples (fewer amplitudes per thread) against the
+    oracle, and the same samples inside batches of 2^19 and 2^20 amplitudes and one of a few more
+    (other tiles, the last one ragged).  Bars as everywhere: 1e-5 on P, 1e-4 on gradients."""
+    gen = torch.Generator().manual_seed(n)
+    th = (torch.rand(3 * n, generator=gen) * 6).tolist()
+    layers = [qandle.AngleEmbedding(name="x", qubits=list(range(n)))]
+    gates = []
+    for d in range(3):
+        for q in range(n):
+            layers.append((qandle.RY, qandle.RX, qandle.RZ)[(q + d) % 3](q, theta=torch.tensor(th[d * n + q]), remapping=None))
+            gates.append((("ry", "rx", "rz")[(q + d) % 3], q, float(torch.tensor(th[d * n + q]))))
+        for q in range(n):
+            layers.append(qandle.CNOT(q, (q + 1 + d) % n))
+            gates.append(("cnot", q, (q + 1 + d) % n))
+    circ = qandle.Circuit(layers + [qandle.MeasureProbability()], num_qubits=n).to(device)
+    few = 3
+    x = torch.rand((1 << 20 >> n) + few, n, generator=gen) * 3
+    w = torch.randn(x.shape, generator=gen)
+
+    def run(rows):
+        with torch.no_grad():
+            P = circ(x=x[:rows].to(device))
+        xx = x[:rows].to(device).requires_grad_(True)
+        (circ(x=xx) * w[:rows].to(device)).sum().backward()
+        return P[:few].cpu().numpy(), xx.grad[:few].cpu().numpy()
+
+    ops = [("embed", "x", list(range(n)), x[:few].double().numpy())] + gates
+    ref = fp64.measure_prob(fp64.simulate(n, ops), n)
+    adj = fp64.adjoint_grads(n, ops, w[:few].double().numpy())[0]
+    for rows in (few, 1 << 19 >> n, 1 << 20 >> n, (1 << 20 >> n) + few):
+        P, gx = run(rows)
+        assert np.abs(P - ref).max() < 1e-5, rows
+        assert np.abs(gx - adj).max() < 1e-4, rows
