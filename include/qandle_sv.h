@@ -248,6 +248,26 @@ int qs_compose_tables(float *utab, float *qtab, const int32_t *recipes,
                       const int32_t *offsets, int nrec, const float *cs,
                       void *stream);
 
+/* One rotation straight from its angle: out = R_P(phi) in on bit `bit` where the
+ * amplitude's bits of cmask are all set (0: everywhere; out may be in).  phi is
+ * device memory: one angle, or with per_sample sample b's at phi[b * phi_stride].
+ * table (NULL: not wanted) gets the half angle's (cos, sin), per sample or one.
+ * What BuiltParametrizedOperator.forward (src/qandle/operators.py:265-298) and,
+ * with cmask, BuiltControlled.forward (:488-506) compute from a dense matrix. */
+int qs_rot_angle(float *out, float *table, const float *in, int64_t B, int n,
+                 int bit, int kind, const float *phi, int64_t phi_stride,
+                 int per_sample, int64_t cmask, int inverse, void *stream);
+/* Its gradients, from that table: gin = R_P(phi)^-1 g (NULL: not wanted) and
+ * dL/dphi = half of Im<g|P|psi> over the amplitudes the control lets through,
+ * psi the rotation's output: gphi[b] with per_sample, else gphi[0] summed over
+ * the batch (NULL: not wanted).  work: qs_rot_backward_work_bytes(B, n) bytes
+ * of device memory (gphi wanted).  Replaces torch autograd of the two above. */
+int64_t qs_rot_backward_work_bytes(int64_t B, int n);
+int qs_rot_backward(float *gin, float *gphi, const float *g, const float *psi,
+                    int64_t B, int n, int bit, int kind, const float *table,
+                    int per_sample, int64_t cmask, void *work,
+                    int64_t work_bytes, void *stream);
+
 /* Everything the passes of one call read besides the state, made in one launch
  * (QS_SETUP_MAX_NAMED: named inputs it takes):
  * - cs: (cos, sin) of every half angle, entries 0..nphi) from phi, then B per

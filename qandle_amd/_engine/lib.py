@@ -40,6 +40,9 @@ SIGNATURES = {
     "qs_pauli_im_work_bytes": (I64, [I64, I32, I32]),
     "qs_pauli_im": (I32, [P, P, P, I64, I32, P, I32, I32, P, I64, P]),
     "qs_pauli_im_controlled": (I32, [P, P, P, I64, I32, P, I32, I32, I64, P, I64, P]),
+    "qs_rot_angle": (I32, [P, P, P, I64, I32, I32, I32, P, I64, I32, I64, I32, P]),
+    "qs_rot_backward_work_bytes": (I64, [I64, I32]),
+    "qs_rot_backward": (I32, [P, P, P, P, I64, I32, I32, I32, P, I32, I64, P, I64, P]),
     "qs_unitary_1q": (I32, [P, P, I64, I32, I32, P, I64, I64, I32, P]),
     "qs_rot_unitaries": (I32, [P, P, I64, I32, P]),
     "qs_mcx": (I32, [P, P, I64, I32, I32, I64, P]),

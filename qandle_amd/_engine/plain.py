@@ -6,7 +6,7 @@ instead (see ``fused.py``).  Backward rules (torch's convention: for a real
 loss the gradient of a complex tensor is dL/dRe + i dL/dIm):
 
 * rotation psi' = U psi:   grad_psi = U^dag g,
-                           dL/dphi = 1/2 Im <g | P | psi'>
+                           dL/dphi = 1/2 Im <g | P | psi'> (both in one kernel, qs_rot_backward)
 * CNOT (self-inverse):     grad_psi = CNOT g
 * AngleEmbedding:          dL/dx_j = 1/2 Im <g | P_j | psi>  (the factors commute)
 * MeasureProbability:      grad_psi = 2 psi * sum_q w_q [bit n-1-q = 0]
@@ -56,49 +56,54 @@ def pauli_im(lam: torch.Tensor, psi: torch.Tensor, n: int, bits, pauli: int) -> 
     return out
 
 
+def _rot_forward(ctx, state, phi, n: int, bit: int, kind: int, cmask: int):
+    state = _c64(state)
+    B = state.shape[0]
+    per_sample = phi.dim() == 1
+    if per_sample and phi.shape[0] != B:
+        raise RuntimeError(f"per-sample angle has {phi.shape[0]} entries, state batch is {B}")
+    phi = phi.detach().to(torch.float32)
+    table = torch.empty(phi.shape + (2,), dtype=torch.float32, device=state.device)
+    out = torch.empty_like(state)
+    L.check(L.load().qs_rot_angle(L.ptr(out), L.ptr(table), L.ptr(state), B, n, bit, kind, L.ptr(phi),
+                                  phi.stride(0) if per_sample else 0, int(per_sample), cmask, 0, L.stream_of(state)),
+            "qs_rot_angle")
+    ctx.save_for_backward(out, table)
+    ctx.meta = (n, bit, kind, per_sample, cmask)
+    return out
+
+
+def _rot_backward(ctx, g):
+    """(gradient of the state, of the angle), each None when not wanted."""
+    out, table = ctx.saved_tensors
+    n, bit, kind, per_sample, cmask = ctx.meta
+    g = _c64(g)
+    B = out.shape[0]
+    lib = L.load()
+    gin = torch.empty_like(g) if ctx.needs_input_grad[0] else None
+    gphi = work = None
+    wb = 0
+    if ctx.needs_input_grad[1]:
+        wb = lib.qs_rot_backward_work_bytes(B, n)
+        work = torch.empty(wb // 4, dtype=torch.float32, device=g.device)
+        gphi = torch.empty(table.shape[:-1], dtype=torch.float32, device=g.device)
+    if gin is not None or gphi is not None:
+        L.check(lib.qs_rot_backward(None if gin is None else L.ptr(gin), None if gphi is None else L.ptr(gphi), L.ptr(g),
+                                    L.ptr(out), B, n, bit, kind, L.ptr(table), int(per_sample), cmask,
+                                    None if work is None else L.ptr(work), wb, L.stream_of(g)), "qs_rot_backward")
+    return gin, gphi
+
+
 class RotFn(torch.autograd.Function):
     """psi' = R_P(phi) psi on one bit position; phi is () (shared) or (B,)."""
 
     @staticmethod
     def forward(ctx, state, phi, n: int, bit: int, kind: int):
-        state = _c64(state)
-        B = state.shape[0]
-        per_sample = phi.dim() == 1
-        if per_sample and phi.shape[0] != B:
-            raise RuntimeError(f"per-sample angle has {phi.shape[0]} entries, state batch is {B}")
-        cs = half_angle_coeffs(phi)
-        out = torch.empty_like(state)
-        L.check(
-            L.load().qs_rot(
-                L.ptr(out), L.ptr(state), B, n, bit, kind, L.ptr(cs), 1 if per_sample else 0, 0,
-                L.stream_of(state),
-            ),
-            "qs_rot",
-        )
-        ctx.save_for_backward(out, cs)
-        ctx.meta = (n, bit, kind, per_sample)
-        return out
+        return _rot_forward(ctx, state, phi, n, bit, kind, 0)
 
     @staticmethod
     def backward(ctx, g):
-        out, cs = ctx.saved_tensors
-        n, bit, kind, per_sample = ctx.meta
-        g = _c64(g)
-        B = g.shape[0]
-        gin = gphi = None
-        if ctx.needs_input_grad[0]:
-            gin = torch.empty_like(g)
-            L.check(
-                L.load().qs_rot(
-                    L.ptr(gin), L.ptr(g), B, n, bit, kind, L.ptr(cs), 1 if per_sample else 0, 1,
-                    L.stream_of(g),
-                ),
-                "qs_rot(inverse)",
-            )
-        if ctx.needs_input_grad[1]:
-            im = pauli_im(g, out, n, [bit], kind)[:, 0] * 0.5
-            gphi = im if per_sample else im.sum()
-        return gin, gphi, None, None, None
+        return *_rot_backward(ctx, g), None, None, None
 
 
 class CnotFn(torch.autograd.Function):
@@ -238,38 +243,11 @@ class ControlledRotFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, state, phi, n: int, bit: int, kind: int, cmask: int):
-        state = _c64(state)
-        B = state.shape[0]
-        if phi.dim() == 1 and phi.shape[0] != B:
-            raise RuntimeError(f"per-sample angle has {phi.shape[0]} entries, state batch is {B}")
-        u = rot_unitaries(half_angle_coeffs(phi), kind)
-        out = _unitary(torch.empty_like(state), state, u, n, bit, cmask, 0)
-        ctx.save_for_backward(out, u)
-        ctx.meta = (n, bit, kind, cmask, phi.dim() == 1)
-        return out
+        return _rot_forward(ctx, state, phi, n, bit, kind, cmask)
 
     @staticmethod
     def backward(ctx, g):
-        out, u = ctx.saved_tensors
-        n, bit, kind, cmask, per_sample = ctx.meta
-        g = _c64(g)
-        gin = gphi = None
-        if ctx.needs_input_grad[0]:
-            gin = _unitary(torch.empty_like(g), g, u, n, bit, cmask, 1)
-        if ctx.needs_input_grad[1]:
-            B = out.shape[0]
-            lib = L.load()
-            wb = lib.qs_pauli_im_work_bytes(B, n, 1)
-            work = torch.empty(max(wb, 4), dtype=torch.uint8, device=out.device)
-            im = torch.empty(B, 1, dtype=torch.float32, device=out.device)
-            L.check(
-                lib.qs_pauli_im_controlled(L.ptr(im), L.ptr(g), L.ptr(out), B, n, L.i32_array([bit]), 1, kind, cmask,
-                                           L.ptr(work), wb, L.stream_of(out)),
-                "qs_pauli_im_controlled",
-            )
-            im = im[:, 0] * 0.5
-            gphi = im if per_sample else im.sum()
-        return gin, gphi, None, None, None, None
+        return *_rot_backward(ctx, g), None, None, None, None
 
 
 class McxFn(torch.autograd.Function):
