@@ -277,7 +277,17 @@ int qs_rot_backward(float *gin, float *gphi, const float *g, const float *psi,
  *   (qs_compose_tables' records): uniform[2i] is the word offset of recipe i
  *   shared by the batch and uniform[2i + 1] its entry in ltab (-1: none), which
  *   gets its matrix-core operands (qs_lane_coeffs; of U^dagger with dagger);
- *   sampled[i] the offsets of the per-sample recipes (B entries each);
+ *   sampled[2i] the offsets of the per-sample recipes (B entries each);
+ * - gtab (NULL: none; ltab is then unused): the real-rotation form
+ *   U = a diag(1, w) R diag(1, g) of those unitaries, 8 floats (t, f, g, w, a) at
+ *   float offset uniform[2i + 1] (sampled[2i + 1], sample b 8 b floats on; -1:
+ *   none), R = [[1, -t], [t, 1]] or, where f is 1, [[t, -1], [1, t]]; and
+ *   ntables + nstables tables of 2^R complex numbers: the table at twords +
+ *   tables[i] holds (float offset, per-sample flag, nf, nn), then nf factors
+ *   (kind, ref, mask) with entry k the product of those whose mask has odd
+ *   parity with k, then nn numbers (mask unused) that multiply every entry;
+ *   kinds QS_FACTOR_*, ref the recipe's word offset or a cs index (ZW, ZNUM: an
+ *   RZ's e^{i phi} and e^{-i phi/2}).  The last nstables are per sample;
  * - efac (NULL: none): product-state factors (qs_product_factors) with the
  *   rotations of recipe lead_words + lead[pos] applied (lead[pos] < 0: none;
  *   lead = NULL: none anywhere); column[pos] is the embedded column of x (row
@@ -286,6 +296,13 @@ int qs_rot_backward(float *gin, float *gphi, const float *g, const float *psi,
  * qs_product_factors and qs_factor_apply one after another.  All pointers are
  * device memory; the struct itself is read on the host during the call. */
 #define QS_SETUP_MAX_NAMED 24
+#define QS_SETUP_MAX_FACTORS 64
+#define QS_FACTOR_G 0
+#define QS_FACTOR_W 1
+#define QS_FACTOR_ZW 2
+#define QS_FACTOR_NUM 3
+#define QS_FACTOR_ZNUM 4
+#define QS_FACTOR_PER_SAMPLE 8
 typedef struct qs_setup_args {
   float *cs;
   float *utab;
@@ -300,16 +317,23 @@ typedef struct qs_setup_args {
   const int32_t *lead_words;
   const int32_t *lead;
   const int32_t *column;
+  float *gtab;
+  const int32_t *twords;
+  const int32_t *tables;
   int64_t B;
   int64_t x_stride;
   int64_t x_step;
   int64_t nphi;
   int64_t nuniform;
   int64_t nsampled;
+  int64_t ntables;
+  int64_t nstables;
   int32_t n;
   int32_t rot;
   int32_t nnamed;
   int32_t dagger;
+  int32_t R;
+  int32_t reserved;
   const float *named[QS_SETUP_MAX_NAMED];
   int64_t named_stride[QS_SETUP_MAX_NAMED];
 } qs_setup_args;

@@ -20,6 +20,7 @@ import numpy as np
 import torch
 
 from .. import config, qw_map
+from . import givens as GV
 from . import lib as L
 from . import planner as PL
 
@@ -347,7 +348,8 @@ def choose_shape(n: int, grad: bool = False, B: int = None):
     """(R, TB) of the specialised kernels for a circuit width and, with ``B``, a batch.
 
     Forward only: from 13 qubits, tiles of 2^13 amplitudes over 256 threads
-    with 32 amplitudes per thread (the fewest passes).  With gradients: from
+    with 32 amplitudes per thread (the fewest passes), or over 512 threads
+    where the unitaries run as rotations (real_rotations).  With gradients: from
     12 qubits, 2^12-amplitude tiles with 16 amplitudes per thread (the adjoint
     holds psi and lambda, and this shape keeps two waves per SIMD).  From 5
     qubits, 2^11-amplitude tiles of one wave; below that, every bit in
@@ -374,6 +376,8 @@ def choose_shape(n: int, grad: bool = False, B: int = None):
             return 5, 6
         return n, DEFAULT_TB
     amps = B << n
+    if n >= 13 and not grad and real_rotations(4, 9, B, n):
+        return 4, 9
     if n <= 11:
         if amps >= 1 << 20:
             return (5, 6) if n == 11 and not grad else (4, 8)
@@ -391,6 +395,23 @@ def choose_shape(n: int, grad: bool = False, B: int = None):
     if grad:
         return (3, 9) if amps < 1 << 21 else (4, 8)
     return (4, 8) if amps < 1 << 20 else (4, 9) if amps < 1 << 22 else (5, 8)
+
+
+def real_rotations(R: int, TB: int, B: int, n: int) -> bool:
+    """Whether compiled forward passes apply their unitaries as real rotations
+    between diagonals (givens) instead of as complex products on the matrix cores.
+
+    The rotations need a quarter of the arithmetic, so they win where a pass is
+    bound by it: a state that fills the chip several times over, 16 amplitudes
+    per thread and four waves per SIMD.  Measured, products at the shape they
+    run best in -> rotations: 20 qubits x 64 2227 -> 1778 us, 24 x 4 3016 ->
+    2500, 20 x 16 (2^24 amplitudes) 667 -> 560, 16 x 128 (2^23) 212 -> 185,
+    13 x 1024 (2^23) 221 -> 194, with gradients 16 x 256 5234 -> 5100.  Below,
+    the longer chain of dependent steps (the diagonals' tables between the
+    rotations) takes back what the arithmetic saves: 17 x 32 (2^22) 196 -> 200,
+    17 x 44 283 -> 285, 16 x 16 (2^20) 176 -> 188, 17 x 11 158 -> 164.  32
+    amplitudes per thread leave two waves per SIMD: 20 x 64 2028, 24 x 4 2793."""
+    return R == 4 and TB >= 8 and (B << n) >= 1 << 23
 
 
 def interpreted_shape(n: int):
@@ -890,7 +911,7 @@ class SetupPlan:
     total: int                # half-angle entries
     nu: int
     nq: int
-    nlane: int                # matrix-core operand entries
+    nlane: int                # floats of the operand table (matrix-core operands, or records and diagonal tables)
     factors: bool
     keep: tuple
 
@@ -898,22 +919,40 @@ class SetupPlan:
         """A call's own argument block with its output tables (device addresses)."""
         a = L.SetupArgs.from_buffer_copy(self.args)
         a.B, a.cs, a.utab, a.ltab, a.efac, a.qtab = B, cs, utab, ltab, efac, qtab
+        if a.R:
+            a.gtab = ltab
         return a
 
 
 def setup_plan(prog: Program, ws: WordSet, lane_index, B: int, device, lead=None, factors: bool = False,
-               dagger: bool = False) -> SetupPlan:
+               dagger: bool = False, kern=None) -> SetupPlan:
     """qs_setup's plan for the recipes of ``ws``: the uniform ones with their entry
-    of ``lane_index`` (jit's lane-table order), the per-sample ones, and with
-    ``factors`` the product-state factors with the leading rotations of ``lead``
+    of ``lane_index`` (jit's lane-table order), the per-sample ones, with ``kern``
+    (forward kernels that have a schedule) the records and diagonal tables of
+    their real-rotation form instead of lane entries, and with ``factors`` the product-state factors with the leading rotations of ``lead``
     (their _leading_tables) applied."""
-    slot = {int(u): k for k, u in enumerate(lane_index or [])}
+    slot = {(int(u), False): k for k, u in enumerate(lane_index or [])}
+    floats = 16 * len(lane_index or [])
+    twords, tables, stables = [], [], []
+    schedule = None if kern is None else kern.schedule
+    if schedule is not None:
+        slot = {key: kern.records[k] for key, k in schedule.records.items()}
+        floats = kern.table_floats
+        where = {u: off for off, u, _ in ws.entries}
+        for at, factors_ in zip(kern.tables, schedule.tables):
+            masked = [f for f in factors_ if f[0].kind not in (GV.NUM, GV.ZNUM)]
+            numbers = [f for f in factors_ if f[0].kind in (GV.NUM, GV.ZNUM)]
+            if len(masked) > L.SETUP_MAX_FACTORS:
+                raise L.EngineError(f"a diagonal table of {len(masked)} factors (at most {L.SETUP_MAX_FACTORS})")
+            ps = any(f.ps for f, _ in factors_)
+            (stables if ps else tables).append(len(twords))
+            twords += [at, int(ps), len(masked), len(numbers)]
+            for f, m in masked + numbers:
+                ref = f.ref if f.kind in (GV.ZW, GV.ZNUM) else where[f.ref]
+                twords += [f.kind | (L.FACTOR_PER_SAMPLE if f.ps else 0), ref, m]
     uniform, sampled = [], []
     for off, u, ps in ws.entries:
-        if ps:
-            sampled.append(off)
-        else:
-            uniform += [off, slot.get(u, -1)]
+        (sampled if ps else uniform).extend([off, slot.get((u, ps), -1)])
     _, _, total, name_off = coefficient_layout(prog, B)
     a = L.SetupArgs()
     column = [-1] * prog.n
@@ -921,15 +960,19 @@ def setup_plan(prog: Program, ws: WordSet, lane_index, B: int, device, lead=None
         a.rot = prog.init[1]
         for j, b in enumerate(prog.init[2]):
             column[b] = j
-    index = L.upload(uniform + sampled + column, torch.int32, device)  # one upload of the three arrays
+    index = L.upload(uniform + sampled + column + tables + stables + twords, torch.int32, device)  # one upload
     keep = [ws.recipes, index]
     a.words, a.uniform = L.ptr(ws.recipes), L.ptr(index)
     a.sampled, a.column = a.uniform + 4 * len(uniform), a.uniform + 4 * (len(uniform) + len(sampled))
-    a.nuniform, a.nsampled, a.n, a.dagger = len(uniform) // 2, len(sampled), prog.n, int(dagger)
+    a.nuniform, a.nsampled, a.n, a.dagger = len(uniform) // 2, len(sampled) // 2, prog.n, int(dagger)
+    if schedule is not None:
+        a.R, a.ntables, a.nstables = schedule.R, len(tables), len(stables)
+        a.tables = a.column + 4 * len(column)
+        a.twords = a.tables + 4 * (len(tables) + len(stables))
     if factors and lead:
         keep += [lead[0], lead[6]]
         a.lead_words, a.lead = L.ptr(lead[0]), L.ptr(lead[6])
-    return SetupPlan(bytes(a), total, ws.nu, ws.nq, len(lane_index or []), factors, tuple(keep))
+    return SetupPlan(bytes(a), total, ws.nu, ws.nq, floats, factors, tuple(keep))
 
 
 def setup_inputs(a, prog: Program, inp: Inputs):
@@ -974,22 +1017,25 @@ def use_jit(n: int, R: int, TB: int) -> bool:
 
 
 def specialised_kernels(prog: Program, pl: PL.Plan, ws: WordSet, B: int, gen_first: bool, fold: bool = False,
-                        load: bool = True):
+                        load: bool = True, exact: tuple = ()):
     """Run-time compiled kernels of this plan's passes (cached on the program);
     with ``fold`` the last pass writes readout partials (readout_fold).
-    ``load`` False only compiles them into the code-object cache."""
+    ``load`` False only compiles them into the code-object cache.  ``exact``:
+    passes whose stored state the caller reads (givens.Schedule)."""
     from . import jit
 
-    opts = getattr(config, "SPECIALISE_OPTIONS", {}) or {}
+    opts = {"givens": real_rotations(pl.R, pl.TB, B, prog.n), **(getattr(config, "SPECIALISE_OPTIONS", {}) or {})}
+    if opts["givens"]:
+        opts.setdefault("waves", 4 if pl.R <= 4 else 2)
 
     def make():
         masks = readout_fold(prog)[1] if fold else None
         return jit.ProgramKernels(ws.host_passes(), prog.n, pl.R, pl.TB, gen_first, prog.measure, readout=masks,
-                                  load=load, **opts)
+                                  load=load, B=B, exact=exact, **opts)
 
     if not load:
         return make()
-    return prog.kept(("jit", id(pl), B, gen_first, prog.measure, fold, tuple(sorted(opts.items()))), make)
+    return prog.kept(("jit", id(pl), B, gen_first, prog.measure, fold, exact, tuple(sorted(opts.items()))), make)
 
 
 def forward_kernels(prog: Program, B: int, R: int, TB: int, cm: PL.CostModel = None, device="cpu",
@@ -1033,8 +1079,9 @@ def warm(prog: Program, B: int, R: int, TB: int, cm: PL.CostModel = None, specia
     fold = folds(prog, jit_on) and not want_state
     pl = get_plan(prog, R, TB, cm, fold)
     ws = pass_words(prog, pl, B, device)
-    kern = specialised_kernels(prog, pl, ws, B, product, fold) if jit_on else None
-    forward_setup(prog, pl, ws, _setup_lanes(kern), B, device, tables, product)
+    exact = (len(ws.passes) - 1,) if want_state or not prog.measure else ()
+    kern = specialised_kernels(prog, pl, ws, B, product, fold, exact=exact) if jit_on else None
+    forward_setup(prog, pl, ws, kern, B, device, tables, product, exact)
 
 
 def _setup_lanes(kern):
@@ -1043,10 +1090,12 @@ def _setup_lanes(kern):
     return kern.lane_index if kern is not None and kern.lanes == "lds" else None
 
 
-def forward_setup(prog: Program, pl: PL.Plan, ws: WordSet, lane_index, B: int, device, lead, factors) -> SetupPlan:
-    """setup_plan of a forward, kept with the program (per plan, batch and device)."""
-    return prog.kept(("setup", id(pl), B, str(device), lane_index is None, lead is None, factors),
-                     lambda: setup_plan(prog, ws, lane_index, B, device, lead, factors))
+def forward_setup(prog: Program, pl: PL.Plan, ws: WordSet, kern, B: int, device, lead, factors, exact=()) -> SetupPlan:
+    """setup_plan of a forward, kept with the program (per plan, batch, device and kernels)."""
+    lane_index = _setup_lanes(kern)
+    kind = None if kern is None else (kern.schedule is not None, lane_index is None)
+    return prog.kept(("setup", id(pl), B, str(device), kind, lead is None, factors, exact),
+                     lambda: setup_plan(prog, ws, lane_index, B, device, lead, factors, kern=kern))
 
 
 def execute(prog: Program, inp: Inputs, cs: torch.Tensor, efac, R: int, TB: int,
@@ -1112,19 +1161,22 @@ class ForwardCall:
     store: typing.Any = None
 
 
-def _forward_call(prog, R, TB, cm, B, device, jit_on, fold, from_state, want_state, lead_tables, tables) -> ForwardCall:
+def _forward_call(prog, R, TB, cm, B, device, jit_on, fold, from_state, want_state, lead_tables, own, kept) -> ForwardCall:
     pl = get_plan(prog, R, TB, cm, fold)
     ws = pass_words(prog, pl, B, device)
     lib = L.load()
-    kern = specialised_kernels(prog, pl, ws, B, not from_state, fold) if jit_on else None
-    plan = forward_setup(prog, pl, ws, _setup_lanes(kern), B, device, lead_tables, not from_state) if tables else None
+    last = len(ws.passes) - 1
+    exact = tuple(range(last + 1)) if kept is None else tuple(sorted(kept))  # states that someone reads
+    if (exact or want_state or not prog.measure) and last not in exact:
+        exact += (last,)
+    kern = specialised_kernels(prog, pl, ws, B, not from_state, fold, exact=exact) if jit_on else None
+    plan = forward_setup(prog, pl, ws, kern, B, device, lead_tables, own and not from_state, exact)
     final = prog.measure and kern is not None and kern.final
     part = 0
     if prog.measure and not final:
         part = (lib.qs_readout_work_bytes if fold else lib.qs_fused_measure_work_bytes)(B, prog.n, R, TB) // 4
-    sizes = (0, 0, 0, part) if plan is None else (max(plan.nu, 1) * 8, max(plan.nlane, 1) * 16,
-                                                  B * prog.n * 4 if plan.factors else 0, part)
-    used = [ws.recipes, ws.offsets, *([] if plan is None else plan.keep), *([w for w, _, _ in ws.passes] if kern is None else [])]
+    sizes = (max(plan.nu, 1) * 8, max(plan.nlane, 16), B * prog.n * 4 if plan.factors else 0, part)
+    used = [ws.recipes, ws.offsets, *plan.keep, *([w for w, _, _ in ws.passes] if kern is None else [])]
     call = ForwardCall(pl, ws, kern, plan, final, sizes, tiles_of(B, prog.n, R + TB), Resident(used))
     npass = len(ws.passes)
     store = [1 if (i + 1 < npass or want_state or not prog.measure) else 0 for i in range(npass)]
@@ -1166,10 +1218,11 @@ def _execute(prog: Program, inp: Inputs, cs, efac, R: int, TB: int, cm=None, wan
     jit_on = use_jit(n, R, TB) if specialise is None else specialise
     fold = folds(prog, jit_on) and (not want_state if fold is None else bool(fold))
     opts = getattr(config, "SPECIALISE_OPTIONS", None)
+    kept = None if checkpoints is not None else tuple(marks or ())
     call = prog.kept(("call", R, TB, (cm or DEFAULT_COST).key(), B, device.index, jit_on, fold, src is None, want_state,
-                      lead_tables is None, own, tuple(sorted(opts.items())) if opts else ()),
+                      lead_tables is None, own, kept, tuple(sorted(opts.items())) if opts else ()),
                      lambda: _forward_call(prog, R, TB, cm, B, device, jit_on, fold, src is not None, want_state,
-                                           lead_tables, own))
+                                           lead_tables, own, kept))
     lib = L.load()
     st = torch._C._cuda_getCurrentRawStream(device.index)
     call.tables.use(st, device)
@@ -1178,28 +1231,22 @@ def _execute(prog: Program, inp: Inputs, cs, efac, R: int, TB: int, cm=None, wan
     work = torch.empty(n_u + n_l + n_f + n_m, dtype=torch.float32, device=device)
     base = L.ptr(work)
     mpart = base + 4 * (n_u + n_l + n_f)
-    args = hold = None
+    hold = None
+    utab, ltab, factors = base, base + 4 * n_u, base + 4 * (n_u + n_l) if n_f else None
     if own:
-        utab, ltab, factors = base, base + 4 * n_u, base + 4 * (n_u + n_l) if n_f else None
         cs = torch.empty(max(call.setup.total, 1), 2, dtype=torch.float32, device=device)
-        args = call.setup.fill(B, L.ptr(cs), utab, ltab, factors)
+    args = call.setup.fill(B, L.ptr(cs), utab, ltab, factors)
+    if own:
         hold = setup_inputs(args, prog, inp)
-    else:
-        table, _ = compose_tables(ws, cs, generators=False)
-        utab, ltab, factors = L.ptr(table), None, None if efac is None else L.ptr(efac)
-    whole = kern is not None and kern.lanes is True  # a lane table of every entry
-    if whole or (not own and kern is not None and kern.lanes):
-        # operands of the matrix-core unitaries, where qs_setup does not make them: every table entry, or
-        # (lanes "lds") each pass's block of the entries it uses, packed pass after pass; none when no pass uses one
-        if own:
-            L.check(lib.qs_setup(ctypes.byref(args), st), "qs_setup")
-            args = None
-        idx = kern.lane_index_on(device) if kern.lanes == "lds" else None
-        if whole or idx is not None:
-            count = ws.nu if idx is None else idx.numel()
-            lanes = torch.empty(max(count, 1) * 16, dtype=torch.float32, device=device)
-            ltab = L.ptr(lanes)
-            L.check(lib.qs_lane_coeffs(ltab, utab, None if idx is None else L.ptr(idx), count, 0, st), "qs_lane_coeffs")
+    elif efac is not None:
+        factors = L.ptr(efac)
+    if kern is not None and kern.lanes is True:
+        # operands of the matrix-core unitaries as a table of every entry
+        L.check(lib.qs_setup(ctypes.byref(args), st), "qs_setup")
+        args = None
+        lanes = torch.empty(max(ws.nu, 1) * 16, dtype=torch.float32, device=device)
+        ltab = L.ptr(lanes)
+        L.check(lib.qs_lane_coeffs(ltab, utab, None, ws.nu, 0, st), "qs_lane_coeffs")
     if out is not None:
         if (out.dtype != torch.complex64 or tuple(out.shape) != (B, 2 ** n) or not out.is_contiguous()
                 or out.device != device):

@@ -29,11 +29,14 @@ C-ABI (``qs_jit_*``) and the code objects are cached on disk by source hash.
 from __future__ import annotations
 
 import ctypes
+import dataclasses
 import hashlib
 import os
 import struct
 import threading
+import typing
 
+from . import givens as GV
 from . import lib as L
 from . import planner as PL
 
@@ -68,7 +71,24 @@ __device__ __forceinline__ float *pinf(float *p) { asm volatile("" : "+s"(p)); r
 // an opaque copy of the thread index: addresses derived from it inside the
 // tile loop are recomputed where they are used instead of being hoisted out
 // of the loop and kept live in vector registers for the whole kernel
+__device__ __forceinline__ float vec(float x) { asm volatile("" : "+v"(x)); return x; }
 __device__ __forceinline__ int pinv(int x) { asm volatile("" : "+v"(x)); return x; }
+// the pieces of a unitary's real-rotation form (_engine/givens.py): a shear, and a factor
+__device__ __forceinline__ void rot_small(float2 &x, float2 &y, float t) {  // [[1, -t], [t, 1]]
+  const float2 p = x, q = y;
+  x = make_float2(fmaf(-t, q.x, p.x), fmaf(-t, q.y, p.y));
+  y = make_float2(fmaf(t, p.x, q.x), fmaf(t, p.y, q.y));
+}
+__device__ __forceinline__ void rot_large(float2 &x, float2 &y, float t) {  // [[t, -1], [1, t]]
+  const float2 p = x, q = y;
+  x = make_float2(fmaf(t, p.x, -q.x), fmaf(t, p.y, -q.y));
+  y = make_float2(fmaf(t, q.x, p.x), fmaf(t, q.y, p.y));
+}
+__device__ __forceinline__ void turn(float2 &x, float c, float s) {
+  const float a = x.x;
+  x.x = fmaf(-s, x.y, c * a);
+  x.y = fmaf(s, a, c * x.y);
+}
 // lane coefficients of a fused unitary (8 floats as int bits at u) for
 // v_mfma_f32_4x4x1f32: A_k = U[lane & 3][k] of the real 4x4 form
 __device__ __forceinline__ void coeffs(const int *up, float (&m)[4]) {
@@ -275,8 +295,13 @@ def pass_source(name: str, words, n: int, R: int, TB: int, lpos, gen: bool, meas
                 prefetch: bool = False, waves: int = None, readout=None, valu_pairs: int = 0,
                 lanes=False, split_pairs: bool = False, lane_off: int = 0, interleave: bool = False,
                 wave_sync: bool = False, stagger: int = 0, stagger_cu: int = 256, direct_store: bool = False,
-                direct_load: bool = False, final: bool = False) -> str:
+                direct_load: bool = False, final: bool = False, givens=None) -> str:
     """HIP source of one specialised forward pass kernel (extern "C" ``name``).
+
+    ``givens``: the pass's steps of givens.Schedule (``GivensPass``); its uniform
+    unitaries then run as real rotations and diagonal tables on the vector ALU
+    instead of complex products on the matrix cores, and the operand options
+    (``lanes``, ``interleave``, ``valu_pairs``) have nothing to do.
 
     ``final`` (a measuring pass whose tile holds whole samples, n <= R + TB): the
     probabilities themselves go to ``A.mpart`` as (B, n), since a sample's only
@@ -401,7 +426,7 @@ def pass_source(name: str, words, n: int, R: int, TB: int, lpos, gen: bool, meas
                   valu_pairs, lanes=lane_k if lanes == "lds" else lanes, interleave=interleave,
                   wave_sync=wave_sync and s + 1 < len(subs) and wave_local(sub, subs[s + 1], TB),
                   tail=[] if direct_store and s == len(subs) - 1 else None, direct_load=direct_load and s == 0,
-                  final=final)
+                  final=final, givens=givens)
     if direct_store:
         e("    __syncthreads();")
         e("  }")
@@ -451,7 +476,7 @@ def async_load_offsets(lpos, R: int, TB: int):
 
 def pass_source_async(name: str, words, n: int, R: int, TB: int, lpos, measure: bool, waves: int = 2,
                       readout=None, lanes="lds", lane_off: int = 0, interleave: int = 4,
-                      wave_sync: bool = True) -> str:
+                      wave_sync: bool = True, givens=None) -> str:
     """HIP source of one specialised forward pass kernel whose HBM reads overlap
     its arithmetic: one persistent workgroup per compute unit holds two tile
     buffers in LDS (2 x 2^(R+TB) amplitudes).  While the sub-passes work on the
@@ -526,7 +551,8 @@ def pass_source_async(name: str, words, n: int, R: int, TB: int, lpos, measure: 
     for si, sub in enumerate(subs):
         _sub_pass(e, sub, si, len(subs), n, R, TB, False, False, measure and si == len(subs) - 1, readout, 0,
                   lanes=lane_k if lanes == "lds" else lanes, interleave=interleave,
-                  wave_sync=wave_sync and si + 1 < len(subs) and wave_local(sub, subs[si + 1], TB), swz_mask=30)
+                  wave_sync=wave_sync and si + 1 < len(subs) and wave_local(sub, subs[si + 1], TB), swz_mask=30,
+                  givens=givens)
     e("    if (A.store) {")
     e("      const int tz = pinv(tid);")
     for it in range(NR // 2):
@@ -559,7 +585,7 @@ def pass_source_async(name: str, words, n: int, R: int, TB: int, lpos, measure: 
 
 def pass_source_tail(name: str, words, n: int, R: int, TB: int, lpos, gen: bool, measure: bool, waves: int = 2,
                      readout=None, lanes="lds", lane_off: int = 0, interleave: int = 4,
-                     wave_sync: bool = True) -> str:
+                     wave_sync: bool = True, givens=None) -> str:
     """HIP source of one specialised forward pass kernel that streams the next
     tile in during the last sub-pass of the current one.  A resident grid (two
     workgroups per compute unit, one tile buffer each, as pass_source) walks
@@ -638,7 +664,7 @@ def pass_source_tail(name: str, words, n: int, R: int, TB: int, lpos, gen: bool,
         _sub_pass(e, sub, si, len(subs), n, R, TB, False, gen and si == 0, measure and last, readout, 0,
                   lanes=lane_k if lanes == "lds" else lanes, interleave=interleave,
                   wave_sync=wave_sync and not last and wave_local(sub, subs[si + 1], TB), swz_mask=30,
-                  tail=prefetch if last else None)
+                  tail=prefetch if last else None, givens=givens)
     if gen:
         e("    __syncthreads();")  # the next tile's first sub-pass writes the tile buffer again
     e("  }")
@@ -647,7 +673,7 @@ def pass_source_tail(name: str, words, n: int, R: int, TB: int, lpos, gen: bool,
 
 
 def pass_source_pipelined(name: str, words, n: int, R: int, TB: int, lpos, gen: bool, measure: bool,
-                          waves: int = None, readout=None, loaders: int = 8) -> str:
+                          waves: int = None, readout=None, loaders: int = 8, givens=None) -> str:
     """HIP source of one specialised forward pass kernel with a load/compute
     pipeline: a persistent workgroup holds two LDS tiles; 2^TB compute
     threads run the sub-passes on one while 2^loaders loader threads store the
@@ -728,7 +754,7 @@ def pass_source_pipelined(name: str, words, n: int, R: int, TB: int, lpos, gen: 
         pipe = {}
         e("    if (cmp) {")
         _sub_pass(e, sub, si, len(subs), n, R, TB, False, gen and si == 0, measure and si == len(subs) - 1, readout,
-                  0, pipe)
+                  0, pipe, givens=givens)
         e("    }")
         e("    __syncthreads();")
         if "finish" in pipe:
@@ -753,7 +779,8 @@ def wave_local(a, b, TB: int) -> bool:
 
 
 def _sub_pass(e, sub, s, nsub, n, R, TB, multi, gen, measure, readout=None, valu_pairs=0, pipe=None, lanes=False,
-              interleave=False, wave_sync=False, swz_mask=31, tail=None, direct_load=False, final=False):
+              interleave=False, wave_sync=False, swz_mask=31, tail=None, direct_load=False, final=False,
+              givens=None):
     """One sub-pass.  ``pipe`` (pipelined kernels): a dict; the tile is
     ``buf[boff + i]``, no closing barrier is emitted, and a measurement's
     cross-wave finish is left in ``pipe["finish"]`` for after the caller's
@@ -817,7 +844,12 @@ def _sub_pass(e, sub, s, nsub, n, R, TB, multi, gen, measure, readout=None, valu
             rmask |= 1 << sub.GP[r]
         e("      if (live) {")
         e(f"        const float2 *E = reinterpret_cast<const float2 *>(A.efac) + sample * {2 * n};")
-        e("        float2 pf = make_float2(1.f, 0.f);")
+        if givens is not None and givens.start:
+            off, span = givens.table(0)
+            e(f"        cint *gs = as_const(reinterpret_cast<const int *>(A.ltab) + {off}{span});")
+            e("        float2 pf = make_float2(__int_as_float(gs[0]), __int_as_float(gs[1]));")
+        else:
+            e("        float2 pf = make_float2(1.f, 0.f);")
         for pos in range(n):
             if not (rmask >> pos) & 1:
                 e(f"        pf = cmul(pf, E[{2 * pos} + ((gbase >> {pos}) & 1)]);")
@@ -844,7 +876,10 @@ def _sub_pass(e, sub, s, nsub, n, R, TB, multi, gen, measure, readout=None, valu
         for line in tail:
             e(line)
     phys = list(range(NR))
-    for si_, (bits, cnots) in enumerate(sub.segments):
+    phases = sub.phases
+    if givens is not None:
+        phys, phases = _emit_givens(e, givens, s)
+    for si_, (bits, cnots) in enumerate(sub.segments if givens is None else []):
         for r, ui, ps in bits:
             off = f"8 * ({ui} + csample)" if ps else f"{8 * ui}"
             e("      {")
@@ -908,10 +943,10 @@ def _sub_pass(e, sub, s, nsub, n, R, TB, multi, gen, measure, readout=None, valu
                         a, b = phys[j], phys[j | (1 << tgt)]
                         e(f"        {{ const float2 x = v[{a}], y = v[{b}]; v[{a}] = cnd ? y : x; v[{b}] = cnd ? x : y; }}")
                 e("      }")
-    if sub.phases:
+    if phases:
         e("      {")
         e("        float pr = 1.f, pi = 0.f;")
-        for pos, ci, fl in sub.phases:
+        for pos, ci, fl in phases:
             if fl & PL.SEG_NOUNAPPLY:
                 continue
             idx = f"({ci} + csample)" if fl & PL.SEG_PER_SAMPLE else f"{ci}"
@@ -944,6 +979,91 @@ def _sub_pass(e, sub, s, nsub, n, R, TB, multi, gen, measure, readout=None, valu
     elif pipe is None:
         e("      __syncthreads();")
     e("    }")
+
+
+@dataclasses.dataclass
+class GivensPass:
+    """One pass's steps of a givens.Schedule, with the float offsets of its records and
+    tables in the buffer that qs_setup fills (A.ltab of the kernels)."""
+
+    schedule: typing.Any
+    index: int
+    records: list
+    tables: list
+
+    @property
+    def start(self) -> bool:
+        return self.index == 0 and self.schedule.start
+
+    def record(self, k: int, ps: bool):
+        return self.records[k], f" + {GV.RECORD} * csample" if ps else ""
+
+    def table(self, t: int):
+        ps = any(f.ps for f, _ in self.schedule.tables[t])
+        return self.tables[t], f" + {2 << self.schedule.R} * csample" if ps else ""
+
+
+def _emit_givens(e, gv: GivensPass, s: int):
+    """The unitaries and CNOTs of sub-pass ``s`` as its schedule's steps.  Records and
+    tables are read through pinned pointers, a table eight entries at a time, so that at
+    most a few blocks of them occupy scalar registers at once.  Returns the register
+    renaming and the phases left to the caller."""
+    steps, phys, left = gv.schedule.steps[gv.index][s]
+    src = "reinterpret_cast<const int *>(A.ltab)"
+    for step in steps:
+        if step[0] == "table":
+            off, span = gv.table(step[1])
+            masks = sorted({m for _f, m in gv.schedule.tables[step[1]]})
+            same = {}  # registers of equal entries: equal parities under every mask
+            for k in step[2]:
+                same.setdefault(tuple(GV.parity(m & k) for m in masks), []).append(k)
+            groups = list(same.values())
+            for g0 in range(0, len(groups), 8):
+                e(f"      {{ cint *g = as_const(pin({src}{span}) + {off});")
+                for q, ks in enumerate(groups[g0:g0 + 8]):
+                    val = [f"__int_as_float(g[{2 * ks[0] + c}])" for c in (0, 1)]
+                    if len(ks) > 1:  # worth two moves: a scalar operand halves the rate of a vector instruction
+                        e(f"        const float x{q} = vec({val[0]}), y{q} = vec({val[1]});")
+                        val = [f"x{q}", f"y{q}"]
+                    for k in ks:
+                        e(f"        turn(v[{k}], {val[0]}, {val[1]});")
+                e("      }")
+        elif step[0] == "rot":
+            off, span = gv.record(step[1], step[2])
+            e(f"      {{ cint *g = as_const(pin({src}{span}) + {off});")
+            # in a vector register: a scalar operand halves the rate of a vector instruction
+            e("        const float t = vec(__int_as_float(g[0]));")
+            for cond, form in (("if (g[1] == 0) ", "small"), ("else ", "large")):
+                e(f"        {cond}{{ " + " ".join(f"rot_{form}(v[{a}], v[{b}], t);" for a, b in step[3]) + " }")
+            e("      }")
+        elif step[0] == "gen":
+            e("      { const int *ut = pin(A.utab);")
+            e(f"        const int *u = ut + 8 * ({step[1]} + csample);")
+            for a, b in step[2]:
+                e(f"        valu_pair(v[{a}], v[{b}], u);")
+            e("      }")
+        elif step[0] == "swap":
+            e(f"      {{ const bool cnd = (gbase >> {step[1]}) & 1;")
+            for a, b in step[2]:
+                e(f"        {{ const float2 x = v[{a}], y = v[{b}]; v[{a}] = cnd ? y : x; v[{b}] = cnd ? x : y; }}")
+            e("      }")
+        else:  # thread
+            e("      { float2 z = make_float2(1.f, 0.f);")
+            for f, pos in step[1]:
+                if f.kind == GV.ZW:
+                    idx = f"({f.ref} + csample)" if f.ps else f"{f.ref}"
+                    e(f"        {{ const float c = __int_as_float(as_const(A.cs)[2 * {idx}]), "
+                      f"d = __int_as_float(as_const(A.cs)[2 * {idx} + 1]), m = c * c + d * d;")
+                    e(f"          if ((gbase >> {pos}) & 1) z = cmul(z, make_float2((c * c - d * d) / m, 2.f * c * d / m)); }}")
+                else:
+                    off, span = gv.record(gv.schedule.record(f.ref, f.ps), f.ps)
+                    at = off + (2 if f.kind == GV.G else 4)
+                    e(f"        {{ cint *g = as_const(pin({src}{span}) + {at});")
+                    e(f"          if ((gbase >> {pos}) & 1) z = cmul(z, make_float2(__int_as_float(g[0]), __int_as_float(g[1]))); }}")
+            for k in range(1 << gv.schedule.R):
+                e(f"        v[{k}] = cmul(z, v[{k}]);")
+            e("      }")
+    return phys, left
 
 
 def _register_offsets(sub, R):
@@ -1628,14 +1748,17 @@ class ProgramKernels:
     MFMA wait states.  ``async_loads`` (pass_source_async: two tile buffers,
     one workgroup per compute unit) and ``tail_prefetch`` (pass_source_tail:
     the next tile streams in during the last sub-pass) are options that give
-    the same bits and measured slower or no faster."""
+    the same bits and measured slower or no faster.  ``givens``: the unitaries
+    as real rotations between diagonals (givens.Schedule; fused.real_rotations
+    says where), for batches of ``B``; ``exact``: passes whose stored state the
+    caller reads."""
 
     def __init__(self, passes, n: int, R: int, TB: int, gen_first: bool, measure: bool,
                  prefetch: bool = False, waves: int = 2, readout=None, valu_pairs: int = 0,
                  grid: str = "full", pipeline: int = 0, lanes="lds", split_pairs: bool = True,
                  interleave: int = 4, wave_sync: bool = True, stagger: int = 0, load: bool = True,
                  async_loads: bool = False, tail_prefetch: bool = False, direct_store=DIRECT_STORE,
-                 direct_load=DIRECT_LOAD_MIN_UNITARIES):
+                 direct_load=DIRECT_LOAD_MIN_UNITARIES, givens: bool = False, B: int = 1, exact=()):
         self.n, self.R, self.TB = n, R, TB
         self.pipelined = bool(pipeline) and n >= R + TB
         self.block = (1 << TB) + ((1 << pipeline) if self.pipelined else 0)
@@ -1643,6 +1766,13 @@ class ProgramKernels:
         # the measuring pass writes the probabilities where a tile holds whole samples
         self.final = measure and n <= R + TB and not (self.pipelined or async_loads or tail_prefetch)
         npass = len(passes)
+        self.schedule = self.records = self.tables = None
+        self.table_floats = 0
+        if givens:
+            lanes = False
+            dec = [PL.decode_pass(w.cpu().numpy() if hasattr(w, "cpu") else w, R, TB) for w, _ns, _lp in passes]
+            self.schedule = GV.Schedule(dec, R, n < R + TB, gen_first, exact)
+            self.records, self.tables, self.table_floats = self.schedule.layout(B)
         self.sources, self.names = [], []
         self.lane_index = []  # utab index of every lane-table entry (lanes == "lds"), pass by pass
         self.persistent = []  # per pass: True when its kernel walks tiles with a resident grid
@@ -1651,6 +1781,7 @@ class ProgramKernels:
             words = w.cpu().numpy() if hasattr(w, "cpu") else w
             nm = f"{KERNEL}_{i}"
             lane_off = len(self.lane_index)
+            gp = GivensPass(self.schedule, i, self.records, self.tables) if givens else None
             if lanes == "lds" and not self.pipelined:
                 self.lane_index += lane_entries(words, R, TB, n < R + TB)
             # direct_load: True, False, or the fewest fused unitaries a pass needs to load directly;
@@ -1667,19 +1798,20 @@ class ProgramKernels:
             if use_tail:
                 self.sources.append(pass_source_tail(nm, words, n, R, TB, lpos, gen_first and i == 0,
                                                      measure and i == npass - 1, waves, readout, lanes, lane_off,
-                                                     interleave, wave_sync))
+                                                     interleave, wave_sync, givens=gp))
             elif use_async:
                 self.sources.append(pass_source_async(nm, words, n, R, TB, lpos, measure and i == npass - 1, waves,
-                                                      readout, lanes, lane_off, interleave, wave_sync))
+                                                      readout, lanes, lane_off, interleave, wave_sync, givens=gp))
             elif self.pipelined:
                 self.sources.append(pass_source_pipelined(nm, words, n, R, TB, lpos, gen_first and i == 0,
-                                                          measure and i == npass - 1, waves, readout, pipeline))
+                                                          measure and i == npass - 1, waves, readout, pipeline,
+                                                          givens=gp))
             else:
                 self.sources.append(pass_source(nm, words, n, R, TB, lpos, gen_first and i == 0,
                                                 measure and i == npass - 1, prefetch, waves, readout, valu_pairs,
                                                 lanes, split_pairs, lane_off, interleave, wave_sync, stagger,
                                                 direct_store=dstore, direct_load=dload,
-                                                final=self.final and i == npass - 1))
+                                                final=self.final and i == npass - 1, givens=gp))
             plain, one = not (use_tail or use_async or self.pipelined), n >= R + TB  # pass_source's gating
             self.direct.append((plain and one and bool(dload) and not (gen_first and i == 0) and not prefetch,
                                 plain and one and bool(dstore)))

@@ -101,15 +101,18 @@ SIGNATURES = {
 
 
 SETUP_MAX_NAMED = 24
+SETUP_MAX_FACTORS = 64
+FACTOR_PER_SAMPLE = 8
 
 
 class SetupArgs(ctypes.Structure):
     """qs_setup_args (include/qandle_sv.h)."""
 
     _fields_ = [(k, ctypes.c_void_p) for k in ("cs", "utab", "qtab", "ltab", "efac", "phi", "x", "words", "uniform",
-                                               "sampled", "lead_words", "lead", "column")]
-    _fields_ += [(k, I64) for k in ("B", "x_stride", "x_step", "nphi", "nuniform", "nsampled")]
-    _fields_ += [(k, ctypes.c_int32) for k in ("n", "rot", "nnamed", "dagger")]
+                                               "sampled", "lead_words", "lead", "column", "gtab", "twords",
+                                               "tables")]
+    _fields_ += [(k, I64) for k in ("B", "x_stride", "x_step", "nphi", "nuniform", "nsampled", "ntables", "nstables")]
+    _fields_ += [(k, ctypes.c_int32) for k in ("n", "rot", "nnamed", "dagger", "R", "reserved")]
     _fields_ += [("named", ctypes.c_void_p * SETUP_MAX_NAMED), ("named_stride", I64 * SETUP_MAX_NAMED)]
 
 

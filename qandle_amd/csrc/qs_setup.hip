@@ -34,22 +34,82 @@ struct SetupCoef {
   }
 };
 
+// U = a D R G (_engine/givens.py): D = diag(1, w), G = diag(1, g), R = [[1, -t],
+// [t, 1]] with a = |u00| p or, where the rotation is past 45 degrees (swap),
+// R = [[t, -1], [1, t]] with a = |u10| p; p, q are the phases of u00, u10,
+// g = conj(p q), w = q conj(p).  Where u00 or u10 is zero its phase cancels out
+// of every product (taken as 1).
+struct Split {
+  C2 g, w, a;
+  double t;
+  bool swap;
+};
+__device__ __forceinline__ Split split_unitary(const M2 &U) {
+  const double c = sqrt(U.a.re * U.a.re + U.a.im * U.a.im), s = sqrt(U.c.re * U.c.re + U.c.im * U.c.im);
+  const C2 p = c > 0 ? C2{U.a.re / c, U.a.im / c} : C2{1, 0}, q = s > 0 ? C2{U.c.re / s, U.c.im / s} : C2{1, 0};
+  const bool swap = s > c;
+  const double m = swap ? s : c;
+  return {cc(cm(p, q)), cm(q, cc(p)), {m * p.re, m * p.im}, (swap ? c : s) / m, swap};
+}
+
 __device__ __forceinline__ void setup_unitary(const qs_setup_args &A, const int32_t *w, int64_t b, int slot,
                                               const SetupCoef &coef) {
   float u[8];
-  store_m2(u, recipe_unitary(w, b, coef));
+  const M2 U = recipe_unitary(w, b, coef);
+  store_m2(u, U);
   float4 *o = reinterpret_cast<float4 *>(A.utab + 8 * (w[0] + b));
   o[0] = make_float4(u[0], u[1], u[2], u[3]);
   o[1] = make_float4(u[4], u[5], u[6], u[7]);
-  if (slot >= 0) {
+  if (slot >= 0 && A.gtab) {
+    const Split x = split_unitary(U);
+    float4 *r = reinterpret_cast<float4 *>(A.gtab + slot + 8 * b);
+    r[0] = make_float4((float)x.t, x.swap ? 1.f : 0.f, (float)x.g.re, (float)x.g.im);
+    r[1] = make_float4((float)x.w.re, (float)x.w.im, (float)x.a.re, (float)x.a.im);
+  } else if (slot >= 0) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) reinterpret_cast<float4 *>(A.ltab)[4 * slot + r] = lane_row(u, r, A.dagger);
   }
   if (A.qtab) recipe_generators(A.qtab, w, b, coef);
 }
 
+// A factor of a diagonal table, or a number: table word (kind, ref, mask).
+__device__ __forceinline__ C2 setup_factor(const qs_setup_args &A, const int32_t *f, int64_t b, const SetupCoef &coef) {
+  const int kind = f[0] & 7;
+  if (kind == QS_FACTOR_ZW || kind == QS_FACTOR_ZNUM) {
+    const float2 v = coef(f[1] + ((f[0] & QS_FACTOR_PER_SAMPLE) ? b : 0));
+    const C2 z = {v.x, -(double)v.y};  // e^{-i phi / 2}, the value at bit 0
+    if (kind == QS_FACTOR_ZNUM) return z;
+    const C2 y = cm(cc(z), cc(z));
+    const double m = z.re * z.re + z.im * z.im;
+    return {y.re / m, y.im / m};
+  }
+  const Split x = split_unitary(recipe_unitary(A.words + f[1], b, coef));
+  return kind == QS_FACTOR_G ? x.g : kind == QS_FACTOR_W ? x.w : x.a;
+}
+
+// One block per table (and sample): entry k is the product of the numbers and of
+// the factors whose mask has odd parity with k.  Every factor is computed once,
+// by its own thread, in double.
+__device__ void setup_table(const qs_setup_args &A, const int32_t *t, int64_t b, const SetupCoef &coef) {
+  __shared__ C2 fac[QS_SETUP_MAX_FACTORS];
+  const int nf = t[2], nn = t[3], lane = threadIdx.x;
+  const int32_t *f = t + 4;
+  if (lane < nf) fac[lane] = setup_factor(A, f + 3 * lane, b, coef);
+  C2 num = {1, 0};
+  for (int k = lane; k < nn; k += 64) num = cm(num, setup_factor(A, f + 3 * (nf + k), b, coef));
+  for (int off = 1; off < 64; off <<= 1) num = cm(num, C2{__shfl_xor(num.re, off, 64), __shfl_xor(num.im, off, 64)});
+  __syncthreads();
+  const int count = 1 << A.R;
+  if (lane < count) {
+    C2 v = num;
+    for (int k = 0; k < nf; ++k)
+      if (__popc(f[3 * k + 2] & lane) & 1) v = cm(v, fac[k]);
+    reinterpret_cast<float2 *>(A.gtab + t[0])[(t[1] ? b * count : 0) + lane] = make_float2((float)v.re, (float)v.im);
+  }
+}
+
 // Thread ranges, each rounded up to whole blocks: half-angle entries, unitaries
-// shared by the batch, per-sample unitaries, factors.  64-thread blocks: the
+// shared by the batch, per-sample unitaries, tables, factors.  64-thread blocks: the
 // items are few and long (double products, sincosf), so they spread over as
 // many compute units as there are blocks.
 __global__ void __launch_bounds__(64) k_setup(qs_setup_args A) {
@@ -72,7 +132,15 @@ __global__ void __launch_bounds__(64) k_setup(qs_setup_args A) {
   }
   const int64_t nps = (int64_t)A.nsampled * A.B;
   if (range(nps)) {
-    if (i < nps) setup_unitary(A, A.words + A.sampled[i / A.B], i % A.B, -1, coef);
+    if (i < nps) setup_unitary(A, A.words + A.sampled[2 * (i / A.B)], i % A.B, A.sampled[2 * (i / A.B) + 1], coef);
+    return;
+  }
+  if (range(64 * A.ntables)) {
+    setup_table(A, A.twords + A.tables[i >> 6], 0, coef);
+    return;
+  }
+  if (range(64 * A.nstables * A.B)) {
+    setup_table(A, A.twords + A.tables[A.ntables + (i >> 6) / A.B], (i >> 6) % A.B, coef);
     return;
   }
   if (!A.efac || i >= A.B * A.n) return;
@@ -125,10 +193,14 @@ int qs_setup(const qs_setup_args *args, void *stream) {
   for (int j = 0; j < A.nnamed; ++j)
     if (!A.named[j]) return QS_EINVAL;
   if (A.nuniform + A.nsampled > 0 && (!A.words || !A.utab || !A.cs)) return QS_EINVAL;
-  if ((A.nuniform > 0 && (!A.uniform || !A.ltab)) || (A.nsampled > 0 && !A.sampled)) return QS_EINVAL;
+  if (A.ntables < 0 || A.nstables < 0 || (A.ntables + A.nstables > 0 && (!A.tables || !A.twords || !A.gtab || !A.words || !A.cs)))
+    return QS_EINVAL;
+  if (A.R < 0 || A.R > 5) return QS_EINVAL;
+  if ((A.nuniform > 0 && (!A.uniform || (!A.ltab && !A.gtab))) || (A.nsampled > 0 && !A.sampled)) return QS_EINVAL;
   if (A.efac && (!A.column || (A.lead && (!A.lead_words || !A.phi)))) return QS_EINVAL;
   const auto blocks = [](int64_t count) { return (count + 63) / 64; };
-  const int64_t g = blocks(ncs) + blocks(A.nuniform) + blocks(A.nsampled * A.B) + (A.efac ? blocks(A.B * A.n) : 0);
+  const int64_t g = blocks(ncs) + blocks(A.nuniform) + blocks(A.nsampled * A.B) + A.ntables + A.nstables * A.B +
+                    (A.efac ? blocks(A.B * A.n) : 0);
   if (g == 0) return QS_OK;
   if (g > 0x7fffffff) return QS_EUNSUPPORTED;
   hipLaunchKernelGGL(k_setup, dim3((unsigned)g), dim3(64), 0, (hipStream_t)stream, A);
