@@ -6,16 +6,17 @@ are exactly those of a single-circuit run), then all circuits share:
 * one coefficient table (all angles -> one ``qs_half_angle_coeffs``),
 * one product-state factor table (``qs_factor_entries``),
 * one state pool, one measurement-partial pool, one words pool,
-* one work-item launch per *level*: level l runs pass l of every circuit that
-  has one, as (descriptor, tile) items in a grid-stride loop; small circuits
-  fit in one tile and finish in level 0,
+* one work-item launch per *level* of a branch (circuits of about as many
+  passes): level l runs pass l of every circuit of the branch that has one, as
+  (descriptor, tile) items in a grid-stride loop; the branches run beside one
+  another on their own streams,
 * one batched MeasureProbability finish.
 
 The backward is the same with adjoint descriptors: level l runs, for every
 circuit, its reverse-sweep step l (its passes in reverse, then the gradient-only
 passes of its embedding), the first step building the co-state from dL/dP.
 
-The level sequence is captured into one hipGraph (torch.cuda.CUDAGraph on
+The launch sequence is captured into one hipGraph (torch.cuda.CUDAGraph on
 ROCm records HIP graph nodes) and replayed: one graph launch per forward or
 forward + backward, independent of the number of circuits.  Levels replace
 the spin-waits a single persistent kernel would need between dependent tiles:
@@ -56,6 +57,42 @@ class _Circ:
     efac_off: int           # float4 entries
     rows: int
     nrot: int
+
+
+# Circuits by their number of passes: the last branch holds every longer one.  A level takes
+# as long as its longest tile, so circuits of few, long passes (one tile of a narrow circuit
+# holds all of its unitaries) and of many, short ones do not share levels: 256 circuits of 4 to
+# 18 qubits have 566 unitaries on the path through the common levels, 317 on the longest branch.
+# Forward + backward of those: 3209 us with common levels, 2382 with the longest passes first, and
+# so in 3 branches 2288, 4 2167, 5 2332, 7 2506 (there are 4 hardware queues); 20 circuits of up to
+# 12 qubits 676 -> 501, 60 of up to 16 1044 -> 859 (7 branches 1167).
+BRANCHES = 4
+
+
+class _Levels:
+    """(descriptor, tile) items level by level; within a level branch by branch, and
+    within a branch the longest pass first (the last workgroups to start are short)."""
+
+    def __init__(self):
+        self.items: typing.Dict[int, list] = {}
+
+    def add(self, level: int, desc: int, ntiles: int, c: "_Circ", words: int):
+        branch = min(len(c.plan.passes), BRANCHES) - 1
+        self.items.setdefault(level, []).extend((branch, -words, desc, t) for t in range(ntiles))
+
+    def build(self, device):
+        """(item tensors, their counts) per level, and per branch its non-empty
+        [(level, first item, count)]."""
+        levels, counts, branches = [], [], [[] for _ in range(BRANCHES)]
+        for level in sorted(self.items):
+            its = np.asarray(sorted(self.items[level]), dtype=np.int32)
+            levels.append(torch.tensor(its[:, 2:].reshape(-1), device=device))
+            counts.append(len(its))
+            for b in range(BRANCHES):
+                at = np.flatnonzero(its[:, 0] == b)
+                if len(at):
+                    branches[b].append((level, int(at[0]), len(at)))
+        return levels, counts, [b for b in branches if b]
 
 
 class UnevenBatch:
@@ -147,6 +184,7 @@ class UnevenBatch:
         self._build_factor_entries()
         self._build_forward()
         self._bw_built = False
+        self._streams = None
         self.graphs = {}
 
     # ------------------------------------------------------------------ helpers
@@ -193,7 +231,7 @@ class UnevenBatch:
         self.fw_tables = fused.upload_tables([], tables, self.device)
         self.fw_utab = torch.empty(max(tables.nu, 1) * 8, dtype=torch.float32, device=self.device)
         descs = bytearray()
-        levels: typing.Dict[int, list] = {}
+        levels = _Levels()
         k = 0
         ntiles_c = L.ctypes.c_int64(0)
         buf = (L.ctypes.c_char * dbytes)()
@@ -210,13 +248,11 @@ class UnevenBatch:
                     self._addr(self.mpart, c.mpart_off) if last else None, 1,
                 )
                 L.check(rc, f"qs_pass_desc(circuit {ci}, pass {pi})")
-                levels.setdefault(pi, []).extend((k, t) for t in range(ntiles_c.value))
+                levels.add(pi, k, ntiles_c.value, c, len(chunks[k]))
                 descs += bytes(buf)
                 k += 1
         self.fw_descs = torch.frombuffer(descs, dtype=torch.uint8).to(self.device)
-        self.fw_levels = [torch.tensor(np.asarray(levels[l], dtype=np.int32).reshape(-1), device=self.device)
-                          for l in sorted(levels)]
-        self.fw_level_items = [len(levels[l]) for l in sorted(levels)]
+        self.fw_levels, self.fw_level_items, self.fw_branches = levels.build(self.device)
         mdescs = bytearray()
         mbuf = (L.ctypes.c_char * mbytes)()
         for ci, c in enumerate(self.circs):
@@ -271,7 +307,7 @@ class UnevenBatch:
         buf = (L.ctypes.c_char * dbytes)()
         ntiles_c = L.ctypes.c_int64(0)
         descs = bytearray()
-        levels: typing.Dict[int, list] = {}
+        levels = _Levels()
         k = 0
         for ci, (c, st) in enumerate(zip(self.circs, steps)):
             for li, (p, wpos, nsub) in enumerate(st):
@@ -284,13 +320,11 @@ class UnevenBatch:
                     self._addr(self.w, c.out_off) if li == 0 else None,
                 )
                 L.check(rc, f"qs_adjoint_desc(circuit {ci}, step {li})")
-                levels.setdefault(li, []).extend((k, t) for t in range(ntiles_c.value))
+                levels.add(li, k, ntiles_c.value, c, len(chunks[k]))
                 descs += bytes(buf)
                 k += 1
         self.bw_descs = torch.frombuffer(descs, dtype=torch.uint8).to(dev)
-        self.bw_levels = [torch.tensor(np.asarray(levels[l], dtype=np.int32).reshape(-1), device=dev)
-                          for l in sorted(levels)]
-        self.bw_level_items = [len(levels[l]) for l in sorted(levels)]
+        self.bw_levels, self.bw_level_items, self.bw_branches = levels.build(dev)
         fbytes = lib.qs_adjoint_finish_desc_bytes()
         fbuf = (L.ctypes.c_char * fbytes)()
         fdescs = bytearray()
@@ -347,6 +381,22 @@ class UnevenBatch:
             out.append(tot)
         return out
 
+    def _run_branches(self, launch, descs, levels, branches):
+        """Every branch's levels in order: the last branch on the caller's stream, the
+        others beside it on their own; the caller's stream waits for all of them."""
+        main = torch.cuda.current_stream(self.device)
+        if self._streams is None:
+            self._streams = [torch.cuda.Stream(self.device) for _ in range(BRANCHES - 1)]
+        side = self._streams[:len(branches) - 1]
+        for s in side:
+            s.wait_stream(main)
+        for s, branch in zip(side + [main], branches):
+            for level, first, cnt in branch:
+                L.check(launch(L.ptr(descs), L.ptr(levels[level]) + 8 * first, cnt, self.R, self.TB, self.grid,
+                               s.cuda_stream), launch.__name__)
+        for s in side:
+            main.wait_stream(s)
+
     def run_forward(self, events=None):
         """Forward of every circuit.  ``events``: optional list; (start, end, bytes)
         HIP events on the launch stream are appended around every level launch."""
@@ -355,16 +405,16 @@ class UnevenBatch:
         L.check(lib.qs_factor_entries(L.ptr(self.efac), L.ptr(self.x), L.ptr(self.entries), self.nentries, st),
                 "qs_factor_entries")
         self._compose(self.fw_tables, self.fw_utab, None, st)
-        nbytes = self.level_bytes() if events is not None else None
-        for lvl, (items, cnt) in enumerate(zip(self.fw_levels, self.fw_level_items)):
-            if events is not None:
+        if events is None:
+            self._run_branches(lib.qs_items_pass, self.fw_descs, self.fw_levels, self.fw_branches)
+        else:
+            for items, cnt, nbytes in zip(self.fw_levels, self.fw_level_items, self.level_bytes()):
                 ev = (torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True))
                 ev[0].record(torch.cuda.current_stream(self.device))
-            L.check(lib.qs_items_pass(L.ptr(self.fw_descs), L.ptr(items), cnt, self.R, self.TB, self.grid, st),
-                    "qs_items_pass")
-            if events is not None:
+                L.check(lib.qs_items_pass(L.ptr(self.fw_descs), L.ptr(items), cnt, self.R, self.TB, self.grid, st),
+                        "qs_items_pass")
                 ev[1].record(torch.cuda.current_stream(self.device))
-                events.append((ev[0], ev[1], nbytes[lvl]))
+                events.append((ev[0], ev[1], nbytes))
         L.check(lib.qs_items_measure_finish(L.ptr(self.m_descs), len(self.circs), self.max_n, st),
                 "qs_items_measure_finish")
 
@@ -375,10 +425,8 @@ class UnevenBatch:
         lib, st = self.lib, self._stream()
         self.psi.copy_(self.state)
         self._compose(self.bw_tables, self.bw_utab, self.bw_qtab, st)
-        for items, cnt in zip(self.bw_levels, self.bw_level_items):
-            L.check(lib.qs_items_adjoint(L.ptr(self.bw_descs), L.ptr(items), cnt, self.R, self.TB, self.grid, st),
-                    "qs_items_adjoint")
-        L.check(lib.qs_items_adjoint_finish(L.ptr(self.f_descs), len(self.circs), 8, st),
+        self._run_branches(lib.qs_items_adjoint, self.bw_descs, self.bw_levels, self.bw_branches)
+        L.check(lib.qs_items_adjoint_finish(L.ptr(self.f_descs), len(self.circs), 32, st),
                 "qs_items_adjoint_finish")
         self.grad_phi.zero_()
         if self.np_rows:
