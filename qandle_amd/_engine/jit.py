@@ -1238,7 +1238,7 @@ def adjoint_source(name: str, words, n: int, R: int, TB: int, lpos, seed: bool,
                    prefetch: bool = False, waves: int = None, readout=None, lanes=False,
                    split_pairs: bool = False, lane_off: int = 0, interleave: bool = False,
                    wave_sync: bool = False, hermitian: bool = False, direct_load: bool = False,
-                   direct_store: bool = False, rows4: bool = True) -> str:
+                   direct_store: bool = False, rows4: bool = True, one_tile: bool = False) -> str:
     """HIP source of one specialised adjoint pass kernel (the adjoint tile of
     qs_adjoint_pass with the pass program compiled in).  ``seed``: the first
     step of the sweep, whose co-state is built from psi and w = dL/dP, with
@@ -1259,12 +1259,16 @@ def adjoint_source(name: str, words, n: int, R: int, TB: int, lpos, seed: bool,
     swaps, the sums landing in lanes 0-3 for one store) instead of one DPP and
     readlane reduction per row: the same additions in the same tree, so the
     gradients are bit for bit the same (4.09-4.17 vs 4.17-4.22 ms for the 15
-    steps at 16 qubits x 256 x 20 layers)."""
+    steps at 16 qubits x 256 x 20 layers).  ``one_tile``: psi and lambda change
+    layout through the same LDS tile, one after the other, for two more waits
+    per sub-pass and half the LDS (AdjointKernels)."""
     K = R + TB
     T, NR = 1 << TB, 1 << R
     multi = n < K
     direct_load = direct_load and not multi and not seed and not prefetch
     direct_store = direct_store and not multi
+    one_tile = one_tile and not prefetch  # a prefetch overwrites the lambda that waits for the tile
+    tl = "tp" if one_tile else "tl"
     subs = PL.decode_adjoint_pass(words, R, TB)
     lpos = [int(x) for x in lpos]
     npos = [] if multi else [p for p in range(n) if p not in lpos]
@@ -1277,7 +1281,8 @@ def adjoint_source(name: str, words, n: int, R: int, TB: int, lpos, seed: bool,
     e(f'extern "C" __global__ void __launch_bounds__({T}){wattr}')
     e(f"{name}(JAdj A) {{")
     e(f"  __shared__ __align__(16) float2 tp[{1 << K}];")
-    e(f"  __shared__ __align__(16) float2 tl[{1 << K}];")
+    if not one_tile:
+        e(f"  __shared__ __align__(16) float2 tl[{1 << K}];")
     lane_k = None
     if lanes == "lds":
         ents = adjoint_lane_entries(words, R, TB)
@@ -1327,8 +1332,15 @@ def adjoint_source(name: str, words, n: int, R: int, TB: int, lpos, seed: bool,
     if lane_k:
         nl = 4 * len(lane_k)
         e(f"    for (int c = ts; c < {nl}; c += {T}) ctab[c] = reinterpret_cast<const float4 *>(A.ltab)[{4 * lane_off} + c];")
-    for it in range(0 if direct_load else NR // 2):
-        e(f"    {{ const int sl = swz(2 * ({it * T} + ts)); const bool sw = sl & 1; const float4 a = pa[{it}];")
+    def stage(it, what, tile):
+        """Amplitude pair ``it`` of psi ("a") or lambda ("b") into its tile."""
+        if split_pairs:
+            e(f"      (void)sw; {tile}[sl] = make_float2({what}.x, {what}.y); {tile}[sl ^ 1] = make_float2({what}.z, {what}.w);")
+        else:
+            e(f"      *reinterpret_cast<float4 *>(&{tile}[sl & ~1]) = make_float4(sw ? {what}.z : {what}.x, "
+              f"sw ? {what}.w : {what}.y, sw ? {what}.x : {what}.z, sw ? {what}.y : {what}.w);")
+
+    def co_state(it):
         if seed:
             # co-state of MeasureProbability for the pair (gi, gi + 1)
             e(f"      const i64 gi = base | g_tid | {goff[it]}LL;")
@@ -1351,45 +1363,60 @@ def adjoint_source(name: str, words, n: int, R: int, TB: int, lpos, seed: bool,
             e("      const float4 b = make_float4(w0 * a.x, w0 * a.y, w1 * a.z, w1 * a.w);")
         else:
             e(f"      const float4 b = pb[{it}];")
-        if split_pairs:
-            e("      (void)sw; tp[sl] = make_float2(a.x, a.y); tp[sl ^ 1] = make_float2(a.z, a.w);")
-            e("      tl[sl] = make_float2(b.x, b.y); tl[sl ^ 1] = make_float2(b.z, b.w); }")
-        else:
-            e("      *reinterpret_cast<float4 *>(&tp[sl & ~1]) = make_float4(sw ? a.z : a.x, sw ? a.w : a.y, sw ? a.x : a.z,"
-              " sw ? a.y : a.w);")
-            e("      *reinterpret_cast<float4 *>(&tl[sl & ~1]) = make_float4(sw ? b.z : b.x, sw ? b.w : b.y, sw ? b.x : b.z,"
-              " sw ? b.y : b.w); }")
+
+    def stage_lambda():
+        for it in range(NR // 2):
+            e(f"    {{ const int sl = swz(2 * ({it * T} + ts)); const bool sw = sl & 1; const float4 a = pa[{it}]; (void)a;")
+            co_state(it)
+            stage(it, "b", tl)
+            e("    }")
+
+    for it in range(0 if direct_load else NR // 2):
+        e(f"    {{ const int sl = swz(2 * ({it * T} + ts)); const bool sw = sl & 1; const float4 a = pa[{it}];")
+        if not one_tile:
+            co_state(it)
+        stage(it, "a", "tp")
+        if not one_tile:
+            stage(it, "b", tl)
+        e("    }")
     e("    __syncthreads();")
     if prefetch:
         e("    { const i64 tn = t + gridDim.x; if (tn < A.ntiles) fetch(tile_base(tn)); }")
     e(f"    const i64 uslot = t * {T >> wlog} + (tid >> {wlog});")
     e(f"    const bool leader = (tid & {(1 << wlog) - 1}) == 0;")
     e(f"    float2 vp[{NR}], vl[{NR}];")
+    if one_tile:
+        e("    int lb8o;  // the tile addresses of the sub-pass that holds lambda")
+    prev = stage_lambda
     for s, sub in enumerate(subs):
-        _adj_sub_pass(e, sub, s, n, R, TB, multi, wlog, lane_k, interleave,
-                      wave_sync and s + 1 < len(subs) and wave_local(sub, subs[s + 1], TB), hermitian,
-                      direct_load=direct_load and s == 0, direct_store=direct_store and s == len(subs) - 1,
-                      rows4=rows4)
+        prev = _adj_sub_pass(e, sub, s, n, R, TB, multi, wlog, lane_k, interleave,
+                             wave_sync and s + 1 < len(subs) and wave_local(sub, subs[s + 1], TB), hermitian,
+                             direct_load=direct_load and s == 0, direct_store=direct_store and s == len(subs) - 1,
+                             rows4=rows4, prev=prev if one_tile else None)
     if direct_store:
         e("    __syncthreads();")
         e("  }")
         e("}")
         return "\n".join(o)
     e("    const int tz = pinv(tid);")
-    for it in range(NR // 2):
-        e(f"    {{ const i64 gi = base | g_tid | {goff[it]}LL; const int sl = swz(2 * ({it * T} + tz)); const bool sw = sl & 1;")
-        cond = "if (gi < total) " if multi else ""
-        if split_pairs:
-            e("      (void)sw; const float2 a0 = tp[sl], a1 = tp[sl ^ 1], b0 = tl[sl], b1 = tl[sl ^ 1];")
-            e(f"      {cond}{{ reinterpret_cast<float4 *>(A.psi)[gi >> 1] = make_float4(a0.x, a0.y, a1.x, a1.y);")
-            e("        reinterpret_cast<float4 *>(A.lam)[gi >> 1] = make_float4(b0.x, b0.y, b1.x, b1.y); } }")
-        else:
-            e("      const float4 a = *reinterpret_cast<const float4 *>(&tp[sl & ~1]);")
-            e("      const float4 b = *reinterpret_cast<const float4 *>(&tl[sl & ~1]);")
-            e(f"      {cond}{{ reinterpret_cast<float4 *>(A.psi)[gi >> 1] = make_float4(sw ? a.z : a.x, sw ? a.w : a.y,"
-              " sw ? a.x : a.z, sw ? a.y : a.w);")
-            e("        reinterpret_cast<float4 *>(A.lam)[gi >> 1] = make_float4(sw ? b.z : b.x, sw ? b.w : b.y,"
-              " sw ? b.x : b.z, sw ? b.y : b.w); } }")
+    parts = [(("psi", "tp", "a"), ("lam", tl, "b"))] if not one_tile else [(("psi", "tp", "a"),), (("lam", tl, "b"),)]
+    for k, part in enumerate(parts):
+        if k:
+            prev()
+        for it in range(NR // 2):
+            e(f"    {{ const i64 gi = base | g_tid | {goff[it]}LL; const int sl = swz(2 * ({it * T} + tz)); "
+              "const bool sw = sl & 1;")
+            for dst, tile, v in part:
+                cond = "if (gi < total) " if multi else ""
+                out = f"reinterpret_cast<float4 *>(A.{dst})[gi >> 1]"
+                if split_pairs:
+                    e(f"      {{ (void)sw; const float2 {v}0 = {tile}[sl], {v}1 = {tile}[sl ^ 1];")
+                    e(f"        {cond}{out} = make_float4({v}0.x, {v}0.y, {v}1.x, {v}1.y); }}")
+                else:
+                    e(f"      {{ const float4 {v} = *reinterpret_cast<const float4 *>(&{tile}[sl & ~1]);")
+                    e(f"        {cond}{out} = make_float4(sw ? {v}.z : {v}.x, sw ? {v}.w : {v}.y, "
+                      f"sw ? {v}.x : {v}.z, sw ? {v}.y : {v}.w); }}")
+            e("    }")
     e("    __syncthreads();")
     e("  }")
     e("}")
@@ -1426,10 +1453,12 @@ def _emit_put(e, expr: str, row: int, wlog: int, indent: str):
 
 
 def _adj_sub_pass(e, sub, s, n, R, TB, multi, wlog, lanes=None, interleave=False, wave_sync=False,
-                  hermitian=False, direct_load=False, direct_store=False, rows4=True):
+                  hermitian=False, direct_load=False, direct_store=False, rows4=True, prev=None):
     """One adjoint sub-pass.  ``direct_load`` (the first sub-pass): psi and lambda
     come straight from the state (psi from ``A.psi_src``) instead of the tiles;
-    ``direct_store`` (the last): they go straight back to the state."""
+    ``direct_store`` (the last): they go straight back to the state.  ``prev``
+    (one tile for psi and lambda): emits what puts lambda into the tile once psi
+    has been taken from it; returns the same for the next sub-pass."""
     NR = 1 << R
     e(f"    {{  // adjoint sub-pass {s}")
     e("      const int tq = pinv(tid);")
@@ -1465,6 +1494,16 @@ def _adj_sub_pass(e, sub, s, n, R, TB, multi, wlog, lanes=None, interleave=False
                 e(f"        vp[{j}] = reinterpret_cast<const float2 *>(A.psi_src)[gbase | {roff[j]}LL]; "
                   f"vl[{j}] = reinterpret_cast<const float2 *>(A.lam)[gbase | {roff[j]}LL];")
         e("      }")
+    elif prev is not None:
+        for j in range(NR):
+            e(f"      vp[{j}] = lds_at(tp, lb8 ^ {8 * swj[j]});")
+        if s == 0:
+            e("      __syncthreads();")
+        prev()
+        if s == 0:
+            e("      __syncthreads();")
+        for j in range(NR):
+            e(f"      vl[{j}] = lds_at(tp, lb8 ^ {8 * swj[j]});")
     else:
         for j in range(NR):
             e(f"      vp[{j}] = lds_at(tp, lb8 ^ {8 * swj[j]}); vl[{j}] = lds_at(tl, lb8 ^ {8 * swj[j]});")
@@ -1611,13 +1650,32 @@ def _adj_sub_pass(e, sub, s, n, R, TB, multi, wlog, lanes=None, interleave=False
                   f"reinterpret_cast<float2 *>(A.lam)[gbase | {roff[j]}LL] = vl[{phys[j]}];")
         e("    }")
         return
+    def sync():
+        if wave_sync:  # the next step keeps the wave-index bits (wave_local)
+            e("      __builtin_amdgcn_fence(__ATOMIC_RELEASE, \"wavefront\"); __builtin_amdgcn_wave_barrier();")
+            e("      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, \"wavefront\");")
+        else:
+            e("      __syncthreads();")
+
+    if prev is not None:
+        # A thread writes the addresses it last read, so only the changes of layout need a wait:
+        # psi written | psi read, lambda written | lambda read, with a barrier at each bar and
+        # one between the two in the middle.
+        for j in range(NR):
+            e(f"      lds_at(tp, lb8 ^ {8 * swj[j]}) = vp[{phys[j]}];")
+        e("      lb8o = lb8;")
+        sync()
+        e("    }")
+
+        def lam():
+            sync()
+            for j in range(NR):
+                e(f"      lds_at(tp, lb8o ^ {8 * swj[j]}) = vl[{phys[j]}];")
+            sync()
+        return lam
     for j in range(NR):
         e(f"      lds_at(tp, lb8 ^ {8 * swj[j]}) = vp[{phys[j]}]; lds_at(tl, lb8 ^ {8 * swj[j]}) = vl[{phys[j]}];")
-    if wave_sync:  # the next step keeps the wave-index bits (wave_local)
-        e("      __builtin_amdgcn_fence(__ATOMIC_RELEASE, \"wavefront\"); __builtin_amdgcn_wave_barrier();")
-        e("      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, \"wavefront\");")
-    else:
-        e("      __syncthreads();")
+    sync()
     e("    }")
 
 
@@ -1868,16 +1926,27 @@ class AdjointKernels:
     amplitude pairs' psi and lambda chains at a time) gives the same bits and
     measured 1.5% slower than the default two chains (4.21-4.24 vs 4.15-4.16 ms).
 
-    Defaults as for ProgramKernels (two waves per SIMD, the U^dagger lane
+    ``one_tile``: a sweep step is arithmetic, LDS traffic and state traffic in
+    turn, and what one workgroup does of one hides under another's.  With a tile
+    each for psi and lambda, 2^12 amplitudes left a compute unit two workgroups;
+    with one tile for both, registers for three waves per SIMD (``waves``) make
+    it three: forward + backward at 16 qubits x 256 x 20 layers 5017 -> 4778 us
+    (two waves per SIMD 4884, four 5009), 14 x 512 1040 -> 939, gradients bit
+    for bit the same; 2^13 amplitudes over 512 threads 7325 -> 5419.
+
+    Defaults as for ProgramKernels (two waves per SIMD elsewhere, the U^dagger lane
     table in LDS, 8-byte pair moves): 18.1 vs 22.2 ms per forward + backward
     at 16 qubits x 256 x 20 layers, 27.5 vs 29.1 ms at 20 qubits x 64,
     gradients bit for bit the same."""
 
     def __init__(self, passes, n: int, R: int, TB: int, seed_first: bool, prefetch: bool = False,
-                 waves: int = 2, readout=None, grid: str = "full", lanes="lds", split_pairs: bool = True,
+                 waves: int = None, readout=None, grid: str = "full", lanes="lds", split_pairs: bool = True,
                  interleave: bool = True, wave_sync: bool = True, hermitian: bool = True,
-                 direct_load=DIRECT_LOAD_MIN_UNITARIES, direct_store=DIRECT_STORE, rows4: bool = True):
+                 direct_load=DIRECT_LOAD_MIN_UNITARIES, direct_store=DIRECT_STORE, rows4: bool = True,
+                 one_tile: bool = True):
         self.block = 1 << TB
+        if waves is None:
+            waves = 3 if one_tile and (R, TB) == (4, 8) else 2
         self.full_grid = grid == "full"
         self.sources, self.names = [], []
         self.lane_index = []
@@ -1895,7 +1964,8 @@ class AdjointKernels:
             dstore = _full_lines(subs_i[-1], R) if direct_store == "auto" else direct_store
             self.sources.append(adjoint_source(nm, words, n, R, TB, lpos, seed_first and i == 0, prefetch, waves,
                                                readout, lanes, split_pairs, lane_off, interleave, wave_sync,
-                                               hermitian, direct_load=dload, direct_store=dstore, rows4=rows4))
+                                               hermitian, direct_load=dload, direct_store=dstore, rows4=rows4,
+                                               one_tile=one_tile))
             self.names.append(nm)
         self.funcs = kernels_for(self.sources, self.names)
         self.grid_cap = [None] * len(self.funcs)
