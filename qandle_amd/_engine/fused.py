@@ -942,8 +942,6 @@ def setup_plan(prog: Program, ws: WordSet, lane_index, B: int, device, lead=None
         for at, factors_ in zip(kern.tables, schedule.tables):
             masked = [f for f in factors_ if f[0].kind not in (GV.NUM, GV.ZNUM)]
             numbers = [f for f in factors_ if f[0].kind in (GV.NUM, GV.ZNUM)]
-            if len(masked) > L.SETUP_MAX_FACTORS:
-                raise L.EngineError(f"a diagonal table of {len(masked)} factors (at most {L.SETUP_MAX_FACTORS})")
             ps = any(f.ps for f, _ in factors_)
             (stables if ps else tables).append(len(twords))
             twords += [at, int(ps), len(masked), len(numbers)]

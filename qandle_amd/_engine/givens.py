@@ -27,6 +27,7 @@ from __future__ import annotations
 
 import dataclasses
 
+from . import lib as L
 from . import planner as PL
 
 # kinds of a diagonal factor (include/qandle_sv.h), the value where its parity is 1 (it is 1
@@ -130,10 +131,14 @@ class Schedule:
         for f, _ in factors:
             if f.kind in (G, W, NUM):
                 self.record(f.ref, f.ps)
-        every = any(f.kind in (NUM, ZNUM) for f, _ in factors)
-        regs = tuple(k for k in range(1 << self.R) if every or any(parity(m & k) for _, m in factors))
-        steps.append(("table", len(self.tables), regs))
-        self.tables.append(list(factors))
+        numbers = [x for x in factors if x[0].kind in (NUM, ZNUM)]
+        masked = [x for x in factors if x[0].kind not in (NUM, ZNUM)]
+        for k in range(0, max(len(masked), 1), L.SETUP_MAX_FACTORS):  # as many as qs_setup multiplies into a table
+            part = masked[k:k + L.SETUP_MAX_FACTORS]
+            regs = tuple(j for j in range(1 << self.R) if numbers or any(parity(m & j) for _, m in part))
+            steps.append(("table", len(self.tables), regs))
+            self.tables.append(part + numbers)
+            numbers = []
 
     def _flush(self, regs: Registers, steps, hit, extra=()):
         """A table of the pending diagonals that ``hit`` picks, with ``extra``."""

@@ -90,6 +90,37 @@ def test_rotations(device, n, B, R, TB, given):
         assert (m - m0).abs().max().item() <= tol
 
 
+def _phases(n, count, gen):
+    """RZ gates on one qubit between CNOTs it controls, on a bit that stays out of the registers
+    until RX mixes it: their diagonals all join one flush."""
+    ops = [("rx", q, 0.3 + q) for q in range(n)]
+    for k in range(count):
+        ops += [("rz", 0, float(torch.rand((), generator=gen))), ("cnot", 0, 1 + k % (n - 1)),
+                ("rx", 1 + (k + 2) % (n - 1), float(torch.rand((), generator=gen)))]
+    return ops + [("rx", q, 0.7 - q) for q in range(n)]
+
+
+@pytest.mark.parametrize("n,count", [(13, 60), (13, 150), (15, 200)])
+def test_many_diagonals(device, n, count):
+    cls = {"rx": qandle.RX, "rz": qandle.RZ}
+    ops = _phases(n, count, torch.Generator().manual_seed(count))
+    layers = [qandle.CNOT(o[1], o[2]) if o[0] == "cnot" else
+              cls[o[0]](o[1], theta=torch.tensor(o[2], dtype=torch.float32), remapping=None) for o in ops]
+    circ = qandle.Circuit(layers + [qandle.MeasureProbability()], num_qubits=n).to(device)
+    prog = fused.lower_circuit(circ.circuit)
+    inp = fused.gather_inputs(prog, circ.circuit, None, {})
+    old = (config.SPECIALISE, config.SPECIALISE_OPTIONS)
+    try:
+        config.SPECIALISE, config.SPECIALISE_OPTIONS = True, {"givens": True}
+        with torch.no_grad():
+            s, _p = fused.execute(prog, inp, fused.build_coeffs(prog, inp), fused.product_factors(prog, inp), 4, 9,
+                                  want_state=True)
+    finally:
+        config.SPECIALISE, config.SPECIALISE_OPTIONS = old
+    ref = fp64.simulate(n, ops)
+    assert np.abs(s.cpu().numpy().reshape(ref.shape) - ref).max() <= len(ops) * 2.0 ** -21
+
+
 @pytest.mark.parametrize("n,B,lines", [(12, 2047, False), (12, 2048, True), (14, 511, False), (14, 513, True)])
 def test_where_the_rotations_run(n, B, lines):
     R, TB = fused.choose_shape(n, False, B)
