@@ -184,7 +184,8 @@ class UnevenBatch:
         self._build_factor_entries()
         self._build_forward()
         self._bw_built = False
-        self._streams = None
+        # made here: a caller's capture of run_forward creates no streams
+        self._streams = [torch.cuda.Stream(dev) for _ in range(BRANCHES - 1)] if dev.type == "cuda" else []
         self.graphs = {}
 
     # ------------------------------------------------------------------ helpers
@@ -385,8 +386,6 @@ class UnevenBatch:
         """Every branch's levels in order: the last branch on the caller's stream, the
         others beside it on their own; the caller's stream waits for all of them."""
         main = torch.cuda.current_stream(self.device)
-        if self._streams is None:
-            self._streams = [torch.cuda.Stream(self.device) for _ in range(BRANCHES - 1)]
         side = self._streams[:len(branches) - 1]
         for s in side:
             s.wait_stream(main)
