@@ -12,8 +12,10 @@ counts as one gate).
 ``qs_pass_<i>``: algorithmic bytes per launch (first pass 8 B per amplitude,
 middle passes 16 B, the measuring last pass 8 B, over the executed schedule)
 divided by the launches' average duration from HIP events on their own
-stream, against 8 TB/s.  ``roofline.mfma`` is the same launches against the
-fp32 matrix-core peak (16 flops per amplitude per fused 2x2 unitary).
+stream, against 8 TB/s.  ``roofline.mfma`` is the same launches' fused 2x2
+unitaries as complex products (16 flops per amplitude) against the fp32
+matrix-core peak; the kernels run them as real rotations (4 flops per
+amplitude) on the vector ALU, so they may pass the matrix cores' rate.
 
 ``extras``: the plain per-gate GPU path, 24 qubits x 4, the adjoint forward +
 backward at 16 qubits x 256 x 20 layers (with the roofline of its ``qs_adj_<i>``
@@ -283,10 +285,10 @@ extern "C" __global__ void __launch_bounds__(256) qs_mfma_probe(float *out, int 
 
 def mfma_sustained(dev, stream):
     """The fp32 matrix-core rate this GPU sustains, measured: 8 independent chains
-    of v_mfma_f32_4x4x1 (the pass kernels' instruction) per wave, with 2 and with
-    8 waves per SIMD (2 is the pass kernels' occupancy).  The published 157.3
-    TFLOP/s assumes the peak engine clock; under matrix-core load the clock runs
-    lower, and this is the rate the pass kernels can approach."""
+    of v_mfma_f32_4x4x1 (the adjoint kernels' instruction, and that of forward
+    passes over smaller states) per wave, with 2 and with 8 waves per SIMD.  The
+    published 157.3 TFLOP/s assumes the peak engine clock; under matrix-core load
+    the clock runs lower."""
     import ctypes
     import struct as st
 
@@ -414,7 +416,7 @@ def main():
     circ = qandle.Circuit(w.layers, num_qubits=n).to(dev)
     x = w.inputs["x"].to(dev)
     prog = fused.lower_circuit(circ.circuit)
-    R, TB = fused.choose_shape(n)
+    R, TB = fused.choose_shape(n, False, B)
 
     def step():
         with torch.no_grad():
@@ -456,6 +458,8 @@ def main():
     sustained = mfma_sustained(dev, stream)
     roof["mfma"] = {"achieved": tflops, "peak": MFMA_F32_PEAK_TFLOPS, "unit": "TFLOP/s",
                     "frac": tflops / MFMA_F32_PEAK_TFLOPS, "alg_flops_per_launch": flops_per_launch,
+                    "executed_as": ("real rotations on the vector ALU (4 flops per amplitude and unitary, and the "
+                                    "diagonals between them)" if fused.real_rotations(R, TB, B, n) else "products"),
                     "fused_unitaries_per_step": units,
                     "sustained_measured": sustained,
                     "frac_of_sustained": tflops / sustained["2_waves_per_simd"]}
@@ -546,7 +550,7 @@ def bench_n24(dev, time_steps, sync):
     settle(fwd, sync)
     t, _ = time_steps(fwd, 5, 2)
     prog = fused.lower_circuit(c.circuit)
-    npass = len(executed_plan(prog, *fused.choose_shape(24)).passes)
+    npass = len(executed_plan(prog, *fused.choose_shape(24, False, 4)).passes)
     nbytes = sum(pass_bytes(4, 24, npass, stores_last=False))
     return {"n24_updates_per_s": w.amplitude_updates() * 5 / t, "n24_ms_per_step": t / 5 * 1e3,
             "n24_hbm_frac": nbytes / (t / 5) / 1e9 / HBM_PEAK_GBS, "n24_passes": npass}

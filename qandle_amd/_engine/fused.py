@@ -404,13 +404,13 @@ def real_rotations(R: int, TB: int, B: int, n: int) -> bool:
     The rotations need a quarter of the arithmetic, so they win where a pass is
     bound by it: a state that fills the chip several times over, 16 amplitudes
     per thread and four waves per SIMD.  Measured, products at the shape they
-    run best in -> rotations: 20 qubits x 64 2227 -> 1778 us, 24 x 4 3016 ->
-    2500, 20 x 16 (2^24 amplitudes) 667 -> 560, 16 x 128 (2^23) 212 -> 185,
+    run best in -> rotations: 20 qubits x 64 2218 -> 1678 us, 24 x 4 2895 ->
+    2321, 20 x 16 (2^24 amplitudes) 667 -> 560, 16 x 128 (2^23) 212 -> 185,
     13 x 1024 (2^23) 221 -> 194, with gradients 16 x 256 5234 -> 5100.  Below,
     the longer chain of dependent steps (the diagonals' tables between the
     rotations) takes back what the arithmetic saves: 17 x 32 (2^22) 196 -> 200,
     17 x 44 283 -> 285, 16 x 16 (2^20) 176 -> 188, 17 x 11 158 -> 164.  32
-    amplitudes per thread leave two waves per SIMD: 20 x 64 2028, 24 x 4 2793."""
+    amplitudes per thread leave two waves per SIMD: 20 x 64 2028 against 1778."""
     return R == 4 and TB >= 8 and (B << n) >= 1 << 23
 
 
@@ -929,8 +929,9 @@ def setup_plan(prog: Program, ws: WordSet, lane_index, B: int, device, lead=None
     """qs_setup's plan for the recipes of ``ws``: the uniform ones with their entry
     of ``lane_index`` (jit's lane-table order), the per-sample ones, with ``kern``
     (forward kernels that have a schedule) the records and diagonal tables of
-    their real-rotation form instead of lane entries, and with ``factors`` the product-state factors with the leading rotations of ``lead``
-    (their _leading_tables) applied."""
+    their real-rotation form instead of lane entries, and with ``factors`` the
+    product-state factors with the leading rotations of ``lead`` (their
+    _leading_tables) applied."""
     slot = {(int(u), False): k for k, u in enumerate(lane_index or [])}
     floats = 16 * len(lane_index or [])
     twords, tables, stables = [], [], []
