@@ -976,8 +976,10 @@ def setup_plan(prog: Program, ws: WordSet, lane_index, B: int, device, lead=None
 
 def setup_inputs(a, prog: Program, inp: Inputs):
     """Puts a call's angle and embedding inputs into its qs_setup argument block;
-    returns the tensors that have to live until the launch."""
-    keep = [inp.phi_param.detach()]
+    returns the tensors that have to live until the launch.  The kernel takes any
+    strides, but reads memory as it is: a lazily negated view (``z.conj().imag``)
+    holds its numbers with the other sign and is materialised first."""
+    keep = [inp.phi_param.detach().resolve_neg()]
     names = list(inp.named)
     if len(names) > L.SETUP_MAX_NAMED:  # one table of all angles
         named = [inp.named[k].detach() for k in names]
@@ -988,12 +990,12 @@ def setup_inputs(a, prog: Program, inp: Inputs):
     a.phi = L.ptr(phi) if a.nphi else a.cs  # no shared angle: any address (it is not read)
     a.nnamed = len(names)
     for j, k in enumerate(names):
-        v = inp.named[k]
+        v = inp.named[k].resolve_neg()
         keep.append(v)
         a.named[j] = L.ptr(v)
         a.named_stride[j] = v.stride(0) if v.dim() else 0
     if a.efac and prog.init[0] == "embed":
-        x = inp.embed_x.detach().to(torch.float32)
+        x = inp.embed_x.detach().to(torch.float32).resolve_neg()
         if x.dim() == 1:
             x = x.unsqueeze(0)
         if x.shape[0] != inp.B:

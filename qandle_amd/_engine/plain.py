@@ -62,7 +62,7 @@ def _rot_forward(ctx, state, phi, n: int, bit: int, kind: int, cmask: int):
     per_sample = phi.dim() == 1
     if per_sample and phi.shape[0] != B:
         raise RuntimeError(f"per-sample angle has {phi.shape[0]} entries, state batch is {B}")
-    phi = phi.detach().to(torch.float32)
+    phi = phi.detach().to(torch.float32).resolve_neg()  # the kernel reads the memory as it is
     table = torch.empty(phi.shape + (2,), dtype=torch.float32, device=state.device)
     out = torch.empty_like(state)
     L.check(L.load().qs_rot_angle(L.ptr(out), L.ptr(table), L.ptr(state), B, n, bit, kind, L.ptr(phi),
