@@ -1082,7 +1082,7 @@ def warm(prog: Program, B: int, R: int, TB: int, cm: PL.CostModel = None, specia
     ws = pass_words(prog, pl, B, device)
     exact = (len(ws.passes) - 1,) if want_state or not prog.measure else ()
     kern = specialised_kernels(prog, pl, ws, B, product, fold, exact=exact) if jit_on else None
-    forward_setup(prog, pl, ws, kern, B, device, tables, product, exact)
+    forward_setup(prog, pl, ws, kern, B, device, tables, product)
 
 
 def _setup_lanes(kern):
@@ -1091,12 +1091,11 @@ def _setup_lanes(kern):
     return kern.lane_index if kern is not None and kern.lanes == "lds" else None
 
 
-def forward_setup(prog: Program, pl: PL.Plan, ws: WordSet, kern, B: int, device, lead, factors, exact=()) -> SetupPlan:
-    """setup_plan of a forward, kept with the program (per plan, batch, device and kernels)."""
-    lane_index = _setup_lanes(kern)
-    kind = None if kern is None else (kern.schedule is not None, lane_index is None)
-    return prog.kept(("setup", id(pl), B, str(device), kind, lead is None, factors, exact),
-                     lambda: setup_plan(prog, ws, lane_index, B, device, lead, factors, kern=kern))
+def forward_setup(prog: Program, pl: PL.Plan, ws: WordSet, kern, B: int, device, lead, factors) -> SetupPlan:
+    """setup_plan of a forward, kept with the program (per plan, batch, device and kernels: the
+    tables are laid out for these kernels, whose own key says all that they depend on)."""
+    return prog.kept(("setup", id(pl), B, str(device), None if kern is None else id(kern), lead is None, factors),
+                     lambda: setup_plan(prog, ws, _setup_lanes(kern), B, device, lead, factors, kern=kern))
 
 
 def execute(prog: Program, inp: Inputs, cs: torch.Tensor, efac, R: int, TB: int,
@@ -1171,7 +1170,7 @@ def _forward_call(prog, R, TB, cm, B, device, jit_on, fold, from_state, want_sta
     if (exact or want_state or not prog.measure) and last not in exact:
         exact += (last,)
     kern = specialised_kernels(prog, pl, ws, B, not from_state, fold, exact=exact) if jit_on else None
-    plan = forward_setup(prog, pl, ws, kern, B, device, lead_tables, own and not from_state, exact)
+    plan = forward_setup(prog, pl, ws, kern, B, device, lead_tables, own and not from_state)
     final = prog.measure and kern is not None and kern.final
     part = 0
     if prog.measure and not final:
