@@ -52,7 +52,7 @@ def _rotation(npairs: int) -> str:
         asm += [f"v_fma_f32 %[r{q}], %[t], %[x{q}], -%[y{q}]", f"v_fma_f32 %[y{q}], %[t], %[y{q}], %[x{q}]"]
     asm.append("2:")
     args = ", ".join(f"float2 &x{k}, float2 &y{k}" for k in range(npairs))
-    outs = ", ".join(f'[r{q}] "=&v"({amp[q][2]}), [y{q}] "+v"({amp[q][1]})' for q in names)
+    outs = ", ".join(f'[r{q}] "=&v"({amp[q][2]}), [y{q}] "+&v"({amp[q][1]})' for q in names)
     ins = ", ".join(f'[x{q}] "v"({amp[q][0]})' for q in names)
     text = "".join(f'    "{line}\\n"\n' for line in asm)
     return (f"__device__ __forceinline__ void rot_pairs{npairs}({args}, float t, int f) {{\n"
@@ -96,7 +96,9 @@ __device__ __forceinline__ int pinv(int x) { asm volatile("" : "+v"(x)); return 
 __device__ __forceinline__ float vec(float x) { asm volatile("" : "+v"(x)); return x; }
 // The pieces of a unitary's real-rotation form (_engine/givens.py): the rotation of amplitude
 // pairs, and a factor (turn).  R = [[1, -t], [t, 1]], or where f is not 0 [[t, -1], [1, t]]; f is
-// the same for every lane.  x' goes to a fresh register and y' to y's own in both forms.  The branch
+// the same for every lane.  x' goes to a fresh register and y' to y's own in both forms; every y is an
+// early clobber too, as it is written while later pairs are still to be read (an x that the
+// compiler knows to be equal to it would otherwise be given y's register).  The branch
 // is inside the block: as control flow of the program both forms' operands stay live together,
 // and the compiler then moves 16 of a rotation's 32 registers where the forms meet again
 // (5690 -> 5040 vector instructions in the 70-unitary pass of 20 qubits x 64; the whole forward
