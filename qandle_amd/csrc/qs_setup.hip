@@ -114,7 +114,7 @@ __device__ void setup_table(const qs_setup_args &A, const int32_t *t, int64_t b,
 // many compute units as there are blocks.
 __global__ void __launch_bounds__(64) k_setup(qs_setup_args A) {
   const SetupCoef coef{A};
-  int64_t i = blockIdx.x * (int64_t)64 + threadIdx.x;
+  int64_t i = (blockIdx.y * (int64_t)gridDim.x + blockIdx.x) * 64 + threadIdx.x;
   const auto range = [&i](int64_t count) {  // true when i falls in the next range
     const int64_t span = (count + 63) / 64 * 64;
     if (i < span) return true;
@@ -202,8 +202,11 @@ int qs_setup(const qs_setup_args *args, void *stream) {
   const int64_t g = blocks(ncs) + blocks(A.nuniform) + blocks(A.nsampled * A.B) + A.ntables + A.nstables * A.B +
                     (A.efac ? blocks(A.B * A.n) : 0);
   if (g == 0) return QS_OK;
-  if (g > 0x7fffffff) return QS_EUNSUPPORTED;
-  hipLaunchKernelGGL(k_setup, dim3((unsigned)g), dim3(64), 0, (hipStream_t)stream, A);
+  // a row of the grid has fewer than 2^32 threads (a block per sample and table passes that
+  // at 64 tables x 2^20 samples); the last row's surplus blocks find no item
+  const int64_t row = g < (1 << 24) ? g : 1 << 24, rows = (g + row - 1) / row;
+  if (rows > 0xffff) return QS_EUNSUPPORTED;
+  hipLaunchKernelGGL(k_setup, dim3((unsigned)row, (unsigned)rows), dim3(64), 0, (hipStream_t)stream, A);
   return launch_status();
 }
 
