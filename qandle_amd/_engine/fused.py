@@ -397,6 +397,13 @@ def choose_shape(n: int, grad: bool = False, B: int = None):
     return (4, 8) if amps < 1 << 20 else (4, 9) if amps < 1 << 22 else (5, 8)
 
 
+# Records and tables of the rotations that a call may hold.  Their places are 32-bit words, and every
+# sample of a circuit with angles of its own has its own: 1984 floats (a quarter of the sample's
+# state) at 12 qubits and 8 re-uploading layers, which reach this at 1.08 million samples.  Such a call's
+# unitaries run as products.
+MAX_TABLE_FLOATS = 2 ** 31 - 1
+
+
 def real_rotations(R: int, TB: int, B: int, n: int) -> bool:
     """Whether compiled forward passes apply their unitaries as real rotations
     between diagonals (givens) instead of as complex products on the matrix cores.
@@ -1025,14 +1032,20 @@ def specialised_kernels(prog: Program, pl: PL.Plan, ws: WordSet, B: int, gen_fir
     passes whose stored state the caller reads (givens.Schedule)."""
     from . import jit
 
-    opts = {"givens": real_rotations(pl.R, pl.TB, B, prog.n), **(getattr(config, "SPECIALISE_OPTIONS", {}) or {})}
-    if opts["givens"]:
-        opts.setdefault("waves", 4 if pl.R <= 4 else 2)
+    given = getattr(config, "SPECIALISE_OPTIONS", {}) or {}
+    opts = {"givens": real_rotations(pl.R, pl.TB, B, prog.n), **given}
 
     def make():
+        kw = dict(opts)
+        if kw["givens"]:
+            kw["givens"] = jit.rotation_schedule(ws.host_passes(), prog.n, pl.R, pl.TB, gen_first, exact)
+            if kw["givens"].layout(B)[2] > MAX_TABLE_FLOATS:
+                kw["givens"] = False
+            elif "waves" not in kw:
+                kw["waves"] = 4 if pl.R <= 4 else 2
         masks = readout_fold(prog)[1] if fold else None
         return jit.ProgramKernels(ws.host_passes(), prog.n, pl.R, pl.TB, gen_first, prog.measure, readout=masks,
-                                  load=load, B=B, exact=exact, **opts)
+                                  load=load, B=B, exact=exact, **kw)
 
     if not load:
         return make()

@@ -1813,6 +1813,12 @@ DIRECT_LOAD_MIN_UNITARIES = 32
 DIRECT_STORE = "auto"
 
 
+def rotation_schedule(passes, n: int, R: int, TB: int, gen_first: bool, exact=()):
+    """givens.Schedule of a forward program's encoded passes."""
+    dec = [PL.decode_pass(w.cpu().numpy() if hasattr(w, "cpu") else w, R, TB) for w, _ns, _lp in passes]
+    return GV.Schedule(dec, R, n < R + TB, gen_first, exact)
+
+
 class ProgramKernels:
     """The specialised kernels of every pass of one encoded forward program.
 
@@ -1828,16 +1834,16 @@ class ProgramKernels:
     one workgroup per compute unit) and ``tail_prefetch`` (pass_source_tail:
     the next tile streams in during the last sub-pass) are options that give
     the same bits and measured slower or no faster.  ``givens``: the unitaries
-    as real rotations between diagonals (givens.Schedule; fused.real_rotations
-    says where), for batches of ``B``; ``exact``: passes whose stored state the
-    caller reads."""
+    as real rotations between diagonals (True, or their schedule if the caller
+    has it already; fused.real_rotations says where), for batches of ``B``;
+    ``exact``: passes whose stored state the caller reads."""
 
     def __init__(self, passes, n: int, R: int, TB: int, gen_first: bool, measure: bool,
                  prefetch: bool = False, waves: int = 2, readout=None, valu_pairs: int = 0,
                  grid: str = "full", pipeline: int = 0, lanes="lds", split_pairs: bool = True,
                  interleave: int = 4, wave_sync: bool = True, stagger: int = 0, load: bool = True,
                  async_loads: bool = False, tail_prefetch: bool = False, direct_store=DIRECT_STORE,
-                 direct_load=DIRECT_LOAD_MIN_UNITARIES, givens: bool = False, B: int = 1, exact=()):
+                 direct_load=DIRECT_LOAD_MIN_UNITARIES, givens=False, B: int = 1, exact=()):
         self.n, self.R, self.TB = n, R, TB
         self.pipelined = bool(pipeline) and n >= R + TB
         self.block = (1 << TB) + ((1 << pipeline) if self.pipelined else 0)
@@ -1849,8 +1855,7 @@ class ProgramKernels:
         self.table_floats = 0
         if givens:
             lanes = False
-            dec = [PL.decode_pass(w.cpu().numpy() if hasattr(w, "cpu") else w, R, TB) for w, _ns, _lp in passes]
-            self.schedule = GV.Schedule(dec, R, n < R + TB, gen_first, exact)
+            self.schedule = rotation_schedule(passes, n, R, TB, gen_first, exact) if givens is True else givens
             self.records, self.tables, self.table_floats = self.schedule.layout(B)
         self.sources, self.names = [], []
         self.lane_index = []  # utab index of every lane-table entry (lanes == "lds"), pass by pass
