@@ -172,15 +172,18 @@ class FusedCircuitFn(torch.autograd.Function):
             base = L.ptr(route.index)
             L.check(lib.qs_gradients(L.ptr(grads), gpart, base + route.first, base + route.rows, base,
                                      route.ngroups, B, NS, slots_per_sample(B, n, R, TB), st), "qs_gradients")
-        g_param = grads[:len(prog.param_slots)] if need_param else None
+        # tensors of their own on the buffer (.data: with version counters of their own, so that one
+        # changed in place leaves what autograd saved of another valid)
+        g_param = grads[:len(prog.param_slots)].data if need_param else None
         g_named = []
         for k, shape in enumerate(ctx.named_shapes):
             lo = route.named.get(ctx.names[k])
-            g_named.append(None if lo is None else grads[lo] if len(shape) == 0 else grads[lo:lo + B].reshape(shape))
+            g_named.append(None if lo is None else grads[lo].data if len(shape) == 0
+                           else grads[lo:lo + B].data.reshape(shape))
         g_embed = None
         if embed:
             lo = route.embed
-            g_embed = grads[lo:lo + len(prog.init[2])] if not batched_x else grads[lo:].reshape(ctx.embed_shape)
+            g_embed = grads[lo:lo + len(prog.init[2])].data if not batched_x else grads[lo:].data.reshape(ctx.embed_shape)
         g_state = None
         if ctx.needs_input_grad[9] and prog.init[0] != "embed":
             shp = ctx.state_shape
