@@ -886,7 +886,8 @@ def _leading_tables(prog: Program, per_pos, B: int, device):
             unit[pos], span[pos], where[pos] = u, (B if ps else 1), tables.offsets[-1]
         recipes = L.upload(tables.recipes(), torch.int32, device)
         offsets = L.upload(tables.offsets, torch.int32, device)
-        return recipes, offsets, tables.count, tables.nu, unit, span, L.upload(where, torch.int32, device)
+        where = L.upload(where, torch.int32, device)
+        return recipes, offsets, tables.count, tables.nu, unit, span, where, Resident([recipes, offsets, where])
 
     return prog.kept(("leading_tables", B, str(device)), make)
 
@@ -896,9 +897,10 @@ def absorb_factors(prog: Program, per_pos, efac: torch.Tensor, cs: torch.Tensor,
     their unitaries are composed per bit position on the device (one recipe
     per position, per sample when an input angle is among them) and applied by
     qs_factor_apply."""
-    recipes, offsets, nrec, nu, unit, span, _ = _leading_tables(prog, per_pos, B, efac.device)
+    recipes, offsets, nrec, nu, unit, span, _, tables = _leading_tables(prog, per_pos, B, efac.device)
     lib = L.load()
     st = L.stream_of(efac)
+    tables.use(st, efac.device)
     utab = torch.empty(max(nu, 1) * 8, dtype=torch.float32, device=efac.device)
     L.check(lib.qs_compose_tables(L.ptr(utab), None, L.ptr(recipes), L.ptr(offsets), nrec, L.ptr(cs), st),
             "qs_compose_tables")
