@@ -245,7 +245,7 @@ def precompile(requests, compiled_from_qubits: int, workers: int = 8) -> int:
 _STREAMS: dict = {}
 
 
-def serving_streams(device, count: int):
+def serving_streams(device, count: int, apart: bool = False):
     """The serving streams of a device: created once per process and shared by
     every engine on it.  HIP maps streams onto a fixed number of hardware
     queues (GPU_MAX_HW_QUEUES, 4 on the machines measured), and a kernel
@@ -253,20 +253,82 @@ def serving_streams(device, count: int):
     queue.  Engines that each took new streams from torch's stream pool put
     the small-request stream on a queue shared with a large-chunk stream often
     enough to move the median latency at 70% load from 3.5-4.5 ms to 120 ms
-    (measured on the serving benchmark's request mix)."""
+    (measured on the serving benchmark's request mix).
+
+    Which queues four streams of the pool get differs from process to process
+    and with the streams taken before.  ``apart`` (for engines with large
+    chunks): streams picked so that the first, the small requests', shares its
+    queue with no other, and only the first may share the default stream's
+    (queues_apart).  The same mix at 7.5 requests/s: p99 1039 ms and mean 47 ms
+    so, against 1609 and 166 with a large stream on the small ones' queue and
+    1707 and 176 with one on the default stream's while every launch waited for
+    that (_launch)."""
     dev = torch.device(device)
-    key = (dev.index if dev.index is not None else torch.cuda.current_device(), int(count))
+    key = (dev.index if dev.index is not None else torch.cuda.current_device(), int(count), apart)
     with _STREAMS_LOCK:
         got = _STREAMS.get(key)
         if got is None:
-            got = _STREAMS[key] = [torch.cuda.Stream(dev) for _ in range(count)]
+            if apart and count > 1:
+                pool = [torch.cuda.Stream(dev) for _ in range(2 * HW_QUEUES)]
+                got = queues_apart(torch.cuda.default_stream(dev), pool, int(count), _waits_behind)
+            else:
+                got = [torch.cuda.Stream(dev) for _ in range(count)]
+            _STREAMS[key] = got
     return got
+
+
+HW_QUEUES = 4       # two of this many streams each find every queue that HIP gives a process by default
+SPIN = 1_000_000    # cycles of a probe (0.4 ms)
+
+
+def _waits_behind(a, b) -> bool:
+    """Whether work on stream b waits for work on a (they share a hardware queue): a kernel on b
+    ends only after a spin that was launched on a before it.  Asked again when it seems so, as
+    a host that is held up between the two sees the same; about 1 ms if they do not share."""
+    x = torch.empty(64, device=a.device)
+    for _ in range(3):
+        ea, eb = torch.cuda.Event(), torch.cuda.Event()
+        with torch.cuda.stream(a):
+            torch.cuda._sleep(SPIN)
+            ea.record(a)
+        with torch.cuda.stream(b):
+            x.fill_(0)
+            eb.record(b)
+        eb.synchronize()
+        behind = ea.query()
+        ea.synchronize()
+        if not behind:
+            return False
+    return True
+
+
+def queues_apart(main, streams, count: int, behind) -> list:
+    """``count`` of ``streams``: the first on ``main``'s hardware queue or one of its own, the
+    others on the remaining queues in turn (``behind(a, b)``: a and b share one).  With too
+    few queues for that, they share what there is."""
+    queues = [[main]]
+    for s in streams:
+        for q in queues:
+            if behind(q[0], s):
+                q.append(s)
+                break
+        else:
+            queues.append([s])
+    shared, others = queues[0][1:], queues[1:]
+    if shared:
+        first, rest = shared[0], others
+    else:
+        first, rest = others[0][0], others[1:]
+    rest = rest or others or [shared]
+    return [first] + [rest[i % len(rest)][i // len(rest) % len(rest[i % len(rest)])] for i in range(count - 1)]
 
 
 _STREAMS_LOCK = threading.Lock()
 
 
 class ServingEngine:
+    _apart = True  # whether the streams are chosen for large chunks (or there are none to choose)
+
     def __init__(self, device, cap_bytes: float = 200e9, streams: int = 4, max_inflight: int = 64,
                  max_wait_s: float = 2.0, compiled_from_qubits: typing.Optional[int] = None,
                  max_chunk_frac: float = 0.25, small_work: float = 1e11, big_share: float = 0.9,
@@ -282,6 +344,7 @@ class ServingEngine:
         self.small_work = small_work
         self.big_cap = int(self.cap * big_share)
         self.streams = serving_streams(self.device, streams)
+        self._apart = False
         self.stream_work = [0] * streams
         self.max_inflight = max_inflight
         self.queue: typing.List[_Chunk] = []
@@ -319,6 +382,9 @@ class ServingEngine:
         while step > 1 and state_footprint(req.n, step, R, TB) > limit:
             step -= 1
         req.chunks = [(lo, min(req.B, lo + step)) for lo in range(0, req.B, step)]
+        if not self._apart and req.work * max(hi - lo for lo, hi in req.chunks) > self.small_work:
+            # large chunks to come: some 20 ms, once per process
+            self.streams, self._apart = serving_streams(self.device, len(self.streams), apart=True), True
         if self.warm:
             cm = fused.DEFAULT_COST if req.compiled else fused.INTERPRETED_COST
             for b in sorted({hi - lo for lo, hi in req.chunks}):
@@ -426,7 +492,11 @@ class ServingEngine:
         req = ch.req
         ch.stream = self.pick_stream(ch)
         s = self.streams[ch.stream]
-        s.wait_stream(torch.cuda.current_stream(self.device))
+        cur = torch.cuda.current_stream(self.device)
+        if not cur.query():
+            # only for work that is there: also an empty wait would pass through the current stream's
+            # hardware queue, behind the large chunks of a stream that shares it
+            s.wait_stream(cur)
         arena = self._arena()
         if arena is not None:
             off = arena.take(ch.state_bytes, top=self.small(ch))
