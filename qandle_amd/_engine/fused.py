@@ -1027,15 +1027,17 @@ def use_jit(n: int, R: int, TB: int) -> bool:
 
 
 def specialised_kernels(prog: Program, pl: PL.Plan, ws: WordSet, B: int, gen_first: bool, fold: bool = False,
-                        load: bool = True, exact: tuple = ()):
+                        load: bool = True, exact: tuple = (), rotations: bool = None):
     """Run-time compiled kernels of this plan's passes (cached on the program);
     with ``fold`` the last pass writes readout partials (readout_fold).
     ``load`` False only compiles them into the code-object cache.  ``exact``:
-    passes whose stored state the caller reads (givens.Schedule)."""
+    passes whose stored state the caller reads (givens.Schedule).  ``rotations``:
+    whether unitaries run as real rotations; None leaves it to real_rotations,
+    whose answer depends on the batch."""
     from . import jit
 
     given = getattr(config, "SPECIALISE_OPTIONS", {}) or {}
-    opts = {"givens": real_rotations(pl.R, pl.TB, B, prog.n), **given}
+    opts = {"givens": real_rotations(pl.R, pl.TB, B, prog.n) if rotations is None else bool(rotations), **given}
 
     def make():
         kw = dict(opts)
@@ -1058,12 +1060,14 @@ def forward_kernels(prog: Program, B: int, R: int, TB: int, cm: PL.CostModel = N
                     load: bool = True):
     """The compiled kernels a measured forward without gradients from a product
     state runs (the program ``execute`` ends up with: leading rotations absorbed,
-    trailing CNOTs folded into the readout), compiled now if the code-object cache
-    does not hold them.  ``device`` only places the encoded words; the kernel
-    sources depend on the program's structure, not on its angles, batch or device,
-    so a worker process can build them ahead of a server that runs them later
-    (``load`` False: compile into the code-object cache without loading them
-    onto a device)."""
+    trailing CNOTs folded into the readout) with its unitaries as products
+    (``rotations`` False), compiled now if the code-object cache does not hold
+    them.  ``device`` only places the encoded words; the kernel sources depend on
+    the program's structure and not on its angles or device, nor, for programs
+    without named inputs, on the batch (a named input's tables lie one after
+    another, one entry per sample), so a worker process can build them ahead of a
+    server that runs them later (``load`` False: compile into the code-object cache
+    without loading them onto a device)."""
     if getattr(config, "ABSORB_LEADING_ROTATIONS", True) and prog.init[0] in ("embed", "input"):
         lead = leading_rotations(prog)
         if lead is not None:
@@ -1071,18 +1075,18 @@ def forward_kernels(prog: Program, B: int, R: int, TB: int, cm: PL.CostModel = N
     fold = folds(prog, True)
     pl = get_plan(prog, R, TB, cm, fold)
     ws = pass_words(prog, pl, B, device)
-    return specialised_kernels(prog, pl, ws, B, True, fold, load=load)
+    return specialised_kernels(prog, pl, ws, B, True, fold, load=load, rotations=False)
 
 
 def warm(prog: Program, B: int, R: int, TB: int, cm: PL.CostModel = None, specialise: bool = None,
-         device="cuda", want_state: bool = False, input_state: bool = False):
+         device="cuda", want_state: bool = False, input_state: bool = False, rotations: bool = None):
     """Builds, uploads and compiles what execute needs for this program and
     batch (the leading rotations' tables, the plan, the pass words and
     fused-unitary recipes, the compiled kernels and the setup launch's plan)
     without launching any work.  A caller that will launch on a busy stream
     (a serving loop) warms ahead, so that execute then does no host work
     that waits for the device.  ``input_state``: the call passes an initial
-    state (no product-state factors)."""
+    state (no product-state factors); ``rotations`` as in execute."""
     n = prog.n
     jit_on = use_jit(n, R, TB) if specialise is None else specialise
     product = not (prog.init[0] in ("input", "amplitude") and input_state)
@@ -1096,7 +1100,7 @@ def warm(prog: Program, B: int, R: int, TB: int, cm: PL.CostModel = None, specia
     pl = get_plan(prog, R, TB, cm, fold)
     ws = pass_words(prog, pl, B, device)
     exact = (len(ws.passes) - 1,) if want_state or not prog.measure else ()
-    kern = specialised_kernels(prog, pl, ws, B, product, fold, exact=exact) if jit_on else None
+    kern = specialised_kernels(prog, pl, ws, B, product, fold, exact=exact, rotations=rotations) if jit_on else None
     forward_setup(prog, pl, ws, kern, B, device, tables, product)
 
 
@@ -1115,7 +1119,7 @@ def forward_setup(prog: Program, pl: PL.Plan, ws: WordSet, kern, B: int, device,
 
 def execute(prog: Program, inp: Inputs, cs: torch.Tensor, efac, R: int, TB: int,
             cm: PL.CostModel = None, want_state: bool = True, checkpoints=None, events=None,
-            specialise: bool = None, fold: bool = None, out: torch.Tensor = None):
+            specialise: bool = None, fold: bool = None, out: torch.Tensor = None, rotations: bool = None):
     """Runs every pass.  Returns (state or None, probs or None).
 
     ``cs``, ``efac``: the half-angle table (build_coeffs) and product-state factors
@@ -1136,8 +1140,13 @@ def execute(prog: Program, inp: Inputs, cs: torch.Tensor, efac, R: int, TB: int,
     interpreting kernels (False; no compilation on first use of a program).
     ``fold``: fold trailing CNOTs into the readout of a measured program
     (readout_fold; compiled kernels only), so that the state left behind is
-    the one before those CNOTs; None folds when the state is not wanted."""
-    psi, probs, _ = _execute(prog, inp, cs, efac, R, TB, cm, want_state, checkpoints, events, specialise, fold, out)
+    the one before those CNOTs; None folds when the state is not wanted.
+
+    ``rotations``: whether compiled passes run their unitaries as real rotations;
+    None leaves it to real_rotations, whose answer depends on the batch (a caller
+    whose results must not depend on it says which)."""
+    psi, probs, _ = _execute(prog, inp, cs, efac, R, TB, cm, want_state, checkpoints, events, specialise, fold, out,
+                             rotations=rotations)
     return psi, probs
 
 
@@ -1176,7 +1185,8 @@ class ForwardCall:
     store: typing.Any = None
 
 
-def _forward_call(prog, R, TB, cm, B, device, jit_on, fold, from_state, want_state, lead_tables, own, kept) -> ForwardCall:
+def _forward_call(prog, R, TB, cm, B, device, jit_on, fold, from_state, want_state, lead_tables, own, kept,
+                  rotations) -> ForwardCall:
     pl = get_plan(prog, R, TB, cm, fold)
     ws = pass_words(prog, pl, B, device)
     lib = L.load()
@@ -1184,7 +1194,9 @@ def _forward_call(prog, R, TB, cm, B, device, jit_on, fold, from_state, want_sta
     exact = tuple(range(last + 1)) if kept is None else tuple(sorted(kept))  # states that someone reads
     if (exact or want_state or not prog.measure) and last not in exact:
         exact += (last,)
-    kern = specialised_kernels(prog, pl, ws, B, not from_state, fold, exact=exact) if jit_on else None
+    kern = None
+    if jit_on:
+        kern = specialised_kernels(prog, pl, ws, B, not from_state, fold, exact=exact, rotations=rotations)
     plan = forward_setup(prog, pl, ws, kern, B, device, lead_tables, own and not from_state)
     final = prog.measure and kern is not None and kern.final
     part = 0
@@ -1203,7 +1215,7 @@ def _forward_call(prog, R, TB, cm, B, device, jit_on, fold, from_state, want_sta
 
 
 def _execute(prog: Program, inp: Inputs, cs, efac, R: int, TB: int, cm=None, want_state=True, checkpoints=None,
-             events=None, specialise=None, fold=None, out=None, marks=None):
+             events=None, specialise=None, fold=None, out=None, marks=None, rotations=None):
     """execute, and the half-angle table it ran with.  ``marks`` (a dict by pass
     index, values filled in): the passes whose output is kept (the later ones run
     in another buffer); a gradient's forward passes it, with or without entries,
@@ -1235,9 +1247,9 @@ def _execute(prog: Program, inp: Inputs, cs, efac, R: int, TB: int, cm=None, wan
     opts = getattr(config, "SPECIALISE_OPTIONS", None)
     kept = None if checkpoints is not None else tuple(marks or ())
     call = prog.kept(("call", R, TB, (cm or DEFAULT_COST).key(), B, device.index, jit_on, fold, src is None, want_state,
-                      lead_tables is None, own, kept, tuple(sorted(opts.items())) if opts else ()),
+                      lead_tables is None, own, kept, rotations, tuple(sorted(opts.items())) if opts else ()),
                      lambda: _forward_call(prog, R, TB, cm, B, device, jit_on, fold, src is not None, want_state,
-                                           lead_tables, own, kept))
+                                           lead_tables, own, kept, rotations))
     lib = L.load()
     st = torch._C._cuda_getCurrentRawStream(device.index)
     call.tables.use(st, device)

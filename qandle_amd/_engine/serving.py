@@ -388,7 +388,7 @@ class ServingEngine:
         if self.warm:
             cm = fused.DEFAULT_COST if req.compiled else fused.INTERPRETED_COST
             for b in sorted({hi - lo for lo, hi in req.chunks}):
-                fused.warm(prog, b, R, TB, cm, req.compiled, self.device)
+                fused.warm(prog, b, R, TB, cm, req.compiled, self.device, rotations=False)
             fused.param_angles(prog, self.device)
         return req
 
@@ -537,7 +537,7 @@ class ServingEngine:
             R, TB = kernel_shape(prog.n, req.compiled)
             cm = fused.DEFAULT_COST if req.compiled else fused.INTERPRETED_COST
             _, probs = fused.execute(prog, inp, None, None, R, TB, cm=cm, want_state=False, specialise=req.compiled,
-                                     out=psi)
+                                     out=psi, rotations=False)  # the same form for every batch
             ch.out = probs
             ch.keep = inp
             ev = torch.cuda.Event()
