@@ -212,13 +212,13 @@ class AdjointCall:
 
 def _adjoint_call(prog, R, TB, cm, B, device, jit_on, fold, embed, seeded) -> AdjointCall:
     n = prog.n
+    rows = len(fused.rotation_rows(prog)) + (len(prog.init[2]) if embed else 0)
+    part = L.work_floats(L.load().qs_adjoint_work_bytes(B, n, R, TB, rows), "qs_adjoint_work_bytes")
     pl = fused.get_plan(prog, R, TB, cm, fold)
     ws, nmain = fused.adjoint_words(prog, pl, B, device, embed, cm)
-    rows = len(fused.rotation_rows(prog)) + (len(prog.init[2]) if embed else 0)
     ntiles, NS = adjoint_geometry(B, n, R, TB)
     kern = specialised_adjoint(prog, pl, ws, B, embed, seeded, fold) if jit_on else None
     plan = fused.setup_plan(prog, ws, None if kern is None else kern.lane_index, B, device, dagger=True)
-    part = L.load().qs_adjoint_work_bytes(B, n, R, TB, rows) // 4
     call = AdjointCall(pl, ws, nmain, kern, plan, (max(plan.nu, 1) * 8, max(plan.nq, 1) * 8, max(plan.nlane, 16),
                                                    max(part, 1)), rows, ntiles, NS,
                        fused.Resident([*plan.keep, *([w for w, _, _ in ws.passes] if kern is None else [])]))

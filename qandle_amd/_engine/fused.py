@@ -1187,9 +1187,11 @@ class ForwardCall:
 
 def _forward_call(prog, R, TB, cm, B, device, jit_on, fold, from_state, want_state, lead_tables, own, kept,
                   rotations) -> ForwardCall:
+    lib = L.load()
+    name = "qs_readout_work_bytes" if fold else "qs_fused_measure_work_bytes"
+    part = L.work_floats(getattr(lib, name)(B, prog.n, R, TB), name)
     pl = get_plan(prog, R, TB, cm, fold)
     ws = pass_words(prog, pl, B, device)
-    lib = L.load()
     last = len(ws.passes) - 1
     exact = tuple(range(last + 1)) if kept is None else tuple(sorted(kept))  # states that someone reads
     if (exact or want_state or not prog.measure) and last not in exact:
@@ -1199,9 +1201,8 @@ def _forward_call(prog, R, TB, cm, B, device, jit_on, fold, from_state, want_sta
         kern = specialised_kernels(prog, pl, ws, B, not from_state, fold, exact=exact, rotations=rotations)
     plan = forward_setup(prog, pl, ws, kern, B, device, lead_tables, own and not from_state)
     final = prog.measure and kern is not None and kern.final
-    part = 0
-    if prog.measure and not final:
-        part = (lib.qs_readout_work_bytes if fold else lib.qs_fused_measure_work_bytes)(B, prog.n, R, TB) // 4
+    if final or not prog.measure:
+        part = 0
     sizes = (max(plan.nu, 1) * 8, max(plan.nlane, 16), B * prog.n * 4 if plan.factors else 0, part)
     used = [ws.recipes, ws.offsets, *plan.keep, *([w for w, _, _ in ws.passes] if kern is None else [])]
     call = ForwardCall(pl, ws, kern, plan, final, sizes, tiles_of(B, prog.n, R + TB), Resident(used))

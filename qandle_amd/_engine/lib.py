@@ -162,6 +162,15 @@ def check(status: int, what: str) -> None:
         raise EngineError(f"{what}: {msg}{extra}")
 
 
+def work_floats(nbytes: int, what: str) -> int:
+    """Floats of a workspace from its size query.  A query answers -1 for a shape the
+    library does not take (a tile outside qs_layout_supported, say): a launch would
+    write past any buffer made for that."""
+    if nbytes < 0:
+        raise EngineError(f"{what}: unsupported shape")
+    return nbytes // 4
+
+
 def stream_of(t: torch.Tensor) -> int:
     """Handle of the current stream of a tensor's device (without building a Stream object)."""
     return torch._C._cuda_getCurrentRawStream(t.device.index)
