@@ -594,10 +594,12 @@ class AngleList:
             return False
         modules = [s.module for s in slots]
         fn = modules[0].remapping
-        if fn not in (qw_map.none, qw_map.tanh) or any("theta" not in m._parameters for m in modules):
+        if fn not in (qw_map.none, qw_map.tanh) or any(m.remapping != fn or "theta" not in m._parameters for m in modules):
             return False
-        shape = tuple(modules[0].theta.shape)
-        return cls(modules, fn, shape) if shape in ((), (1,)) else False
+        shape = modules[0].theta.shape
+        if tuple(shape) not in ((), (1,)) or any(m.theta.shape != shape for m in modules):
+            return False  # a gather that fails costs a call more than the general one
+        return cls(modules, fn, tuple(shape))
 
     def gather(self, device):
         """(S,) float32 remapped angles on ``device``, or None when the modules changed."""
@@ -631,6 +633,7 @@ def param_angles(prog: Program, device) -> torch.Tensor:
         phi = prog.angles.gather(device)
         if phi is not None:
             return phi
+        prog.angles = AngleList.of(prog)  # the modules changed
     params = [prog.slots[i] for i in prog.param_slots]
     if not params:
         return torch.zeros(0, dtype=torch.float32, device=device)
