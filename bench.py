@@ -12,10 +12,10 @@ counts as one gate).
 ``qs_pass_<i>``: algorithmic bytes per launch (first pass 8 B per amplitude,
 middle passes 16 B, the measuring last pass 8 B, over the executed schedule)
 divided by the launches' average duration from HIP events on their own
-stream, against 8 TB/s.  ``roofline.mfma`` is the same launches' fused 2x2
-unitaries as complex products (16 flops per amplitude) against the fp32
-matrix-core peak; the kernels run them as real rotations (4 flops per
-amplitude) on the vector ALU, so they may pass the matrix cores' rate.
+stream, against 8 TB/s.  ``roofline.fp32`` is the arithmetic of the same
+launches' fused 2x2 unitaries as the kernels run them (real rotations, 4 flops
+per amplitude; complex products, 16, where the state is small) against the fp32
+peak, which the vector pipes and the matrix cores share.
 
 ``extras``: the plain per-gate GPU path, 24 qubits x 4, the adjoint forward +
 backward at 16 qubits x 256 x 20 layers (with the roofline of its ``qs_adj_<i>``
@@ -42,7 +42,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
-MFMA_F32_PEAK_TFLOPS = 157.3  # dense fp32 matrix-core peak of one MI355X
+FP32_PEAK_TFLOPS = 157.3  # fp32 peak of one MI355X, on the vector pipes and on the matrix cores
 _T0 = time.perf_counter()
 
 
@@ -453,16 +453,15 @@ def main():
         per_pass.append({"us": sum(ds) / len(ds), "unitaries": struct[i][0], "sub_passes": struct[i][1],
                          "alg_bytes": pbytes[i]})
     units = sum(u for u, _ in struct)
-    flops_per_launch = units / npass * B * 2 ** n * 16
+    rotations = fused.use_jit(n, R, TB) and fused.real_rotations(R, TB, B, n)
+    flops_per_launch = units / npass * B * 2 ** n * (4 if rotations else 16)
     tflops = flops_per_launch / (roof["avg_launch_us"] / 1e6) / 1e12
-    sustained = mfma_sustained(dev, stream)
-    roof["mfma"] = {"achieved": tflops, "peak": MFMA_F32_PEAK_TFLOPS, "unit": "TFLOP/s",
-                    "frac": tflops / MFMA_F32_PEAK_TFLOPS, "alg_flops_per_launch": flops_per_launch,
-                    "executed_as": ("real rotations on the vector ALU (4 flops per amplitude and unitary, and the "
-                                    "diagonals between them)" if fused.real_rotations(R, TB, B, n) else "products"),
-                    "fused_unitaries_per_step": units,
-                    "sustained_measured": sustained,
-                    "frac_of_sustained": tflops / sustained["2_waves_per_simd"]}
+    roof["fp32"] = {"achieved": tflops, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": tflops / FP32_PEAK_TFLOPS,
+                    "unitary_flops_per_launch": flops_per_launch,
+                    "executed_as": ("real rotations on the vector pipes, 4 flops per amplitude and unitary (the "
+                                    "diagonals between them are not counted)" if rotations
+                                    else "complex products on the matrix cores, 16 flops per amplitude and unitary"),
+                    "fused_unitaries_per_step": units, "matrix_core_sustained": mfma_sustained(dev, stream)}
     roof["per_pass"] = per_pass
     traffic = None
     tpath = os.path.join(ROOT, "profiles", "traffic_fused_pass_n20_b64.json")

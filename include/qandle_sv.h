@@ -61,7 +61,8 @@ int qs_embed_angle(float *out, const float *x, int64_t B, int n,
                    const int32_t *bits, int d, int rot, int64_t x_stride,
                    void *stream);
 
-/* One rotation on bit position `bit`: out = U psi (out may equal in).
+/* One rotation on bit position `bit`: out = U psi (out may equal in).  For
+ * callers that hold a (cos, sin) table; the package calls qs_rot_angle.
  * Coefficients for sample b are cs[2*(b*cs_stride)], cs_stride 0 = shared,
  * 1 = one (cos, sin) pair per sample.  inverse != 0 applies U^dagger.
  * Replaces BuiltParametrizedOperator.forward `state @ M` / the batched bmm
@@ -112,8 +113,9 @@ int qs_pauli_im(float *out, const float *lam, const float *psi, int64_t B,
 
 /* qs_pauli_im restricted to the amplitudes whose bits cmask are all 1 (the
  * generator P (x) |1..1><1..1| of a controlled rotation; cmask must not hold
- * a bit of `bits`).  Gradient of a Controlled rotation
- * (src/qandle/operators.py:488-506) in the plain path. */
+ * a bit of `bits`): gradient of a Controlled rotation
+ * (src/qandle/operators.py:488-506) on its own, several bits at a time;
+ * qs_rot_backward makes it with the state's gradient. */
 int qs_pauli_im_controlled(float *out, const float *lam, const float *psi,
                            int64_t B, int n, const int32_t *bits, int d,
                            int pauli, int64_t cmask, void *work,
@@ -137,7 +139,8 @@ int qs_unitary_1q(float *out, const float *in, int64_t B, int n, int bit,
                   void *stream);
 
 /* u[8k..8k+8) = R_kind(phi_k) from cs (cos, sin of phi_k / 2), the matrices of
- * src/qandle/operators.py:368-395 in the column convention. */
+ * src/qandle/operators.py:368-395 in the column convention: rotations as
+ * qs_unitary_1q's u (the package's controlled rotations are qs_rot_angle's). */
 int qs_rot_unitaries(float *u, const float *cs, int64_t count, int kind,
                      void *stream);
 
@@ -391,7 +394,8 @@ int qs_readout_finish(float *out, const float *mpart, int64_t B, int n, int R,
  * MeasureProbability co-state from psi while loading instead of reading lam:
  * lam = 2 psi * sum_q seed_w[b, q] [bit n-1-q = 0], seed_w (B, n) float32.
  * qs_adjoint_finish turns the partials into
- * out[r, b] = dL/dphi_r for sample b and tot[r] = sum over b.
+ * out[r, b] = dL/dphi_r for sample b and tot[r] = sum over b (qs_gradients
+ * below, which the package calls, into the gradients themselves).
  * ------------------------------------------------------------------------- */
 int64_t qs_adjoint_work_bytes(int64_t B, int n, int R, int TB, int rows);
 int qs_adjoint_pass(float *psi, float *lam, int64_t B, int n, int R, int TB,

@@ -363,10 +363,40 @@ def choose_shape(n: int, grad: bool = False, B: int = None):
     calls, old shape -> this one: 8 qubits x 32 forward 23.6 -> 18.4 us, with
     gradients 112 -> 51; 11 x 75 29.5 -> 23.0 and 138 -> 83; 14 x 4 46 -> 36
     and 152 -> 120; 16 x 12 64 -> 55 and 215 -> 202; 13 x 200 with gradients
-    (one 2^13 tile per sample) 221 -> 169.  Where the lines lie, both sides:
-    10 x 3000 (2^21.6) R = 3 41.2, R = 4 36.5 us; 16 x 50 (2^21.6) forward
-    R = 4 106.0, R = 5 107.3; 18 x 8 (2^21) with gradients, ladder circuit,
-    R = 3 277, R = 4 258."""
+    (one 2^13 tile per sample) 221 -> 169.
+
+    Where the lines lie, both sides (device time in us of captured calls, 5
+    layers of RX, RY, RZ and a CNOT ladder; this rule's shape first).  The lines
+    were set before these were taken: "!" marks those where the other side is
+    the faster one, by a factor of two in the batch at most.
+
+    * forward, up to 10 qubits, (3, 7) | 2^20 | (4, 8): 8 x 2048 23.1 against
+      23.5, 8 x 4096 24.6 against 26.7; 10 x 512 27.9 against 27.2 (!), 10 x
+      1024 28.0 against 31.6
+    * 11 qubits, (3, 8) | 2^20 | (5, 6): 11 x 256 26.5 against (3, 7) 34.3 and
+      (4, 8) 29.2; 11 x 512 35.4 against (4, 8) 30.1 (!), 11 x 2048 50.7
+      against 52.7, 11 x 4096 83.4 against 68.3 (!, rotations)
+    * 12 qubits, (4, 8): 12 x 16 28.8 against (3, 9) 31.9, 12 x 256 30.2
+      against 33.8, 12 x 1024 54.2 against 61.3
+    * 13 qubits, (5, 8): 13 x 1 37.8 against (3, 9) 34.5 (!), 13 x 64 38.3
+      against 36.9 (!), 13 x 256 40.9 against 54.6, 13 x 512 56.1 against (4, 9) 58.3
+    * from 14, (3, 8) | 2^19 | (4, 8) | 2^20 | (4, 9) | 2^22 | (5, 8): 14 x 16 33.0
+      against 35.8, 14 x 32 37.2 against 35.1 (!), 16 x 8 38.9 against 40.3;
+      14 x 64 50.6 against (4, 8) 40.7 (!), 16 x 16 54.0 against 42.6 (!), 16 x
+      32 61.7 against 57.7 (!); 16 x 64 88.5 against (4, 9) 84.9 (!), 17 x 32
+      (hea) with (4, 9) 196
+    * gradients, (2, 6) to 8 qubits, (3, n - 3) to 11: 8 x 32 72.1 against (3, 6)
+      82.5, 5 x 32 61.0 against 56.2 (!); 9 x 64 79.7 against (2, 6) 87.9, 11 x
+      75 101.9 against 118.8; | 2^20 | (4, 8): 8 x 4096 124.8 against (2, 6) 117.4
+      (!), 8 x 8192 155.0 against 175.5; 11 x 512 144.2 against (3, 8) 127.5 (!)
+    * gradients, 12 qubits, (3, 9) | 2^20 | (4, 8): 12 x 128 123.3 against 132.4,
+      12 x 256 147.4 against 133.7 (!), 12 x 512 182.4 against 215.7
+    * gradients, 13 qubits, (3, 8) | 2^19 | (3, 9) | 2^20 | (4, 9): 13 x 32 126.6
+      against 135.8, 13 x 64 139.7 against 134.0 (!), 13 x 128 174.0 against
+      160.8 (!), 13 x 256 189.2 against 233.1
+    * gradients, from 14, (3, 8) | 2^19 | (3, 9) | 2^21 | (4, 8): 14 x 16 132.4
+      against 142.2, 14 x 32 149.9 against 139.0 (!), 16 x 16 185.8 against
+      209.8; 14 x 128 236.1 against 224.4 (!), 16 x 32 257.0 against 268.0"""
     if B is None or n < 5:
         if n >= 13 and not grad:
             return 5, 8

@@ -11,7 +11,7 @@ per register, a table multiplication.  A diagonal waits (``carry``) while its
 bit is not a register, past CNOTs that it controls, past sub-passes and
 passes, until its bit is rotated again; one that is never rotated again before
 a measurement is dropped.  The numbers a (R grows an amplitude by at most
-sqrt(2)) join a table after every NUMBERS unitaries; the last ones start the
+sqrt(2)) join a table once NUMBERS of them wait; the last ones start the
 generated state.
 
 The matrix cores do not help here: gfx950 runs v_mfma_f32_4x4x1f32 on the
@@ -35,7 +35,9 @@ from . import planner as PL
 # unitary's a, an RZ's e^{-i phi / 2}
 G, W, ZW, NUM, ZNUM = 0, 1, 2, 3, 4
 RECORD = 8    # floats per unitary: t, the form, g, w, a
-NUMBERS = 64  # unitaries between two applications of their numbers: amplitudes grow by at most 2^32
+# Numbers that wait before they are applied.  They are looked at where a segment starts, so up to
+# NUMBERS - 1 + R unitaries may pass: amplitudes grow by at most 2^34 (R <= 5)
+NUMBERS = 64
 
 
 @dataclasses.dataclass(frozen=True)

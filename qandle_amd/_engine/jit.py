@@ -1907,20 +1907,6 @@ class ProgramKernels:
             self.funcs = []
         self.grid_cap = [None] * len(self.funcs)
         self.lanes = lane_mode(lanes, self.pipelined)
-        self._lane_idx = {}
-
-    def lane_index_on(self, device):
-        """The lane-table index list as a device int32 tensor (None unless lanes == "lds")."""
-        if self.lanes != "lds" or not self.lane_index:
-            return None
-        key = str(device)
-        t = self._lane_idx.get(key)
-        if t is None:
-            import torch
-
-            t = L.upload(self.lane_index, torch.int32, device)
-            self._lane_idx[key] = t
-        return t
 
     def grid(self, i: int, ntiles: int) -> int:
         """Workgroups of pass i's launch."""
@@ -1995,18 +1981,6 @@ class AdjointKernels:
             self.names.append(nm)
         self.funcs = kernels_for(self.sources, self.names)
         self.grid_cap = [None] * len(self.funcs)
-
-    def lane_index_on(self, device):
-        """The U^dagger lane-table index list as a device int32 tensor (None when unused)."""
-        if not self.lane_index:
-            return None
-        key = str(device)
-        cache = self.__dict__.setdefault("_lane_idx", {})
-        if key not in cache:
-            import torch
-
-            cache[key] = L.upload(self.lane_index, torch.int32, device)
-        return cache[key]
 
     def grid(self, i: int, ntiles: int) -> int:
         """Workgroups of step i's launch."""

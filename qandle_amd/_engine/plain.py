@@ -195,15 +195,6 @@ class MeasureProbFn(torch.autograd.Function):
 # positions that must all be 1 for the gate to act (0 = uncontrolled).
 # ----------------------------------------------------------------------------
 
-def rot_unitaries(cs: torch.Tensor, kind: int) -> torch.Tensor:
-    """(..., 8) float32 column-convention R_kind from (..., 2) (cos, sin) of phi/2."""
-    u = torch.empty(cs.shape[:-1] + (8,), dtype=torch.float32, device=cs.device)
-    count = cs.numel() // 2
-    if count:
-        L.check(L.load().qs_rot_unitaries(L.ptr(u), L.ptr(cs), count, kind, L.stream_of(cs)), "qs_rot_unitaries")
-    return u
-
-
 def _unitary(out, src, u, n: int, bit: int, cmask: int, dagger: int):
     B = src.shape[0]
     per_sample = u.dim() == 2

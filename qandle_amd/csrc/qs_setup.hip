@@ -9,7 +9,8 @@
 // device time and six of the eleven launches of an 8-qubit batch-32 forward.
 // Here every item recomputes the angles it needs from the inputs (a sincosf or
 // three) instead of reading another kernel's table, so one grid covers all of
-// them with no order between its threads; the values are the same bit for bit.
+// them with no order between its threads; the tables are the same bit for bit, the
+// factors to a few ulp (the compiler contracts their products differently).
 #include "qs_compose.h"
 #include "qs_program.h"
 

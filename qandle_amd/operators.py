@@ -4,8 +4,8 @@ Same class names, constructor contracts, ``build()`` protocol, ``named``
 dispatch flag, ``state_dict`` keys (``...theta``) and registry
 (``BUILT_CLASS_RELATION`` with its ``.T`` inverse) as the reference.  What
 changed is underneath: no operator holds a 2^n x 2^n gate-matrix cache.  A
-rotation is applied by the HIP kernel ``qs_rot`` from two scalars
-(cos(phi/2), sin(phi/2)); CNOT is the exact permutation ``qs_cnot``.  Inside a
+rotation is applied by the HIP kernel ``qs_rot_angle`` straight from its angle
+(cos(phi/2), sin(phi/2) on the way); CNOT is the exact permutation ``qs_cnot``.  Inside a
 ``Circuit`` the operators are not called one by one at all: the circuit lowers
 them to a program for the fused engine.
 """
