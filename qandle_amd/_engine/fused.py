@@ -624,12 +624,12 @@ class AngleList:
             return False
         modules = [s.module for s in slots]
         fn = modules[0].remapping
-        if fn not in (qw_map.none, qw_map.tanh) or any(m.remapping != fn or "theta" not in m._parameters for m in modules):
+        if fn not in (qw_map.none, qw_map.tanh) or [m.remapping for m in modules] != [fn] * len(modules):
             return False
-        shape = modules[0].theta.shape
-        if tuple(shape) not in ((), (1,)) or any(m.theta.shape != shape for m in modules):
+        shapes = {None if t is None else t.shape for t in (m._parameters.get("theta") for m in modules)}
+        if len(shapes) > 1 or not shapes <= {torch.Size(()), torch.Size((1,))}:
             return False  # a gather that fails costs a call more than the general one
-        return cls(modules, fn, tuple(shape))
+        return cls(modules, fn, tuple(shapes.pop()))
 
     def gather(self, device):
         """(S,) float32 remapped angles on ``device``, or None when the modules changed."""
@@ -675,7 +675,8 @@ def param_angles(prog: Program, device) -> torch.Tensor:
         if sl.kind == "param" and sl.module.remapping in elementwise:
             groups.setdefault(sl.module.remapping, []).append(k)
         elif sl.kind == "param":
-            pieces.append(sl.module.remapping(sl.module.theta).reshape(-1)[:1].to(device=device, dtype=torch.float32))
+            v = sl.module.remapping(sl.module.theta).reshape(-1)[:1].to(device=device, dtype=torch.float32)
+            pieces.append(v.resolve_neg())
             order.append([k])
         else:
             values.append(k)
@@ -1021,7 +1022,7 @@ def setup_inputs(a, prog: Program, inp: Inputs):
     returns the tensors that have to live until the launch.  The kernel takes any
     strides, but reads memory as it is: a lazily negated view (``z.conj().imag``)
     holds its numbers with the other sign and is materialised first."""
-    keep = [inp.phi_param.detach().resolve_neg()]
+    keep = [inp.phi_param.detach()]  # param_angles' own tensor
     names = list(inp.named)
     if len(names) > L.SETUP_MAX_NAMED:  # one table of all angles
         named = [inp.named[k].detach() for k in names]
@@ -1032,12 +1033,16 @@ def setup_inputs(a, prog: Program, inp: Inputs):
     a.phi = L.ptr(phi) if a.nphi else a.cs  # no shared angle: any address (it is not read)
     a.nnamed = len(names)
     for j, k in enumerate(names):
-        v = inp.named[k].resolve_neg()
+        v = inp.named[k]
+        if v.is_neg():
+            v = v.resolve_neg()
         keep.append(v)
         a.named[j] = L.ptr(v)
         a.named_stride[j] = v.stride(0) if v.dim() else 0
     if a.efac and prog.init[0] == "embed":
-        x = inp.embed_x.detach().to(torch.float32).resolve_neg()
+        x = inp.embed_x.detach().to(torch.float32)
+        if x.is_neg():
+            x = x.resolve_neg()
         if x.dim() == 1:
             x = x.unsqueeze(0)
         if x.shape[0] != inp.B:
