@@ -278,13 +278,13 @@ def serving_streams(device, count: int, apart: bool = False):
 
 
 HW_QUEUES = 4       # two of this many streams each find every queue that HIP gives a process by default
-SPIN = 1_000_000    # cycles of a probe (0.4 ms)
+SPIN = 2_000_000    # cycles of a probe (0.8 ms)
 
 
 def _waits_behind(a, b) -> bool:
     """Whether work on stream b waits for work on a (they share a hardware queue): a kernel on b
     ends only after a spin that was launched on a before it.  Asked again when it seems so, as
-    a host that is held up between the two sees the same; about 1 ms if they do not share."""
+    a host that is held up between the two sees the same; one spin if they do not share."""
     x = torch.empty(64, device=a.device)
     for _ in range(3):
         ea, eb = torch.cuda.Event(), torch.cuda.Event()
