@@ -62,6 +62,8 @@ def _rot_forward(ctx, state, phi, n: int, bit: int, kind: int, cmask: int):
     per_sample = phi.dim() == 1
     if per_sample and phi.shape[0] != B:
         raise RuntimeError(f"per-sample angle has {phi.shape[0]} entries, state batch is {B}")
+    if phi.device != state.device:
+        raise L.EngineError(f"the angle is on {phi.device}, the state on {state.device}")
     phi = phi.detach().to(torch.float32).resolve_neg()  # the kernel reads the memory as it is
     table = torch.empty(phi.shape + (2,), dtype=torch.float32, device=state.device)
     out = torch.empty_like(state)
